@@ -350,6 +350,19 @@ static void fit_ewald(SysDev& d) {
   }
 }
 
+// Tiles of a system's pair list: pairs inside the cutoff at the mean density, 30 to
+// a tile of 64 lanes.
+static double pair_tiles_estimate(int n, const double L[3], double rc) {
+  const double rho = n / (L[0] * L[1] * L[2]);
+  return 0.5 * n * (4.0 / 3.0 * kPi * rc * rc * rc * rho) / 30.0;
+}
+
+// Systems of up to this many tiles keep an entry list in the mixed form (reason at
+// k_pair_entry): up to about 2,700 atoms at a cutoff of 10.  Larger ones are bound by
+// the pair kernel's arithmetic and atomics, of which the groups need a third less.
+constexpr double ENTRY_TILES = 16384.0;
+static int has_entry_list(int mixed, double tiles) { return mixed && tiles < ENTRY_TILES; }
+
 int System::alloc_device() {
   const HostTopo& h = topo;
   SysDev& d = dv;
@@ -517,6 +530,7 @@ int System::alloc_device() {
   FZ_TRY(dalloc(&d.mF, (size_t)3 * n));
   FZ_TRY(dalloc(&snap, (size_t)9 * n + (F_NSLOT * sizeof(int) + 7) / 8));
   d.snap = snap;
+  d.entry_list = has_entry_list(mixed, pair_tiles_estimate(n, par.box, par.cutoff));
   return set_column_grid(par.column_grid[0], par.column_grid[1], 1.0);
 }
 
@@ -548,13 +562,6 @@ static size_t rnd256(size_t b) { return (std::max<size_t>(1, b) + 255) & ~(size_
 // search each I cluster with several waves: more waves in flight)
 static int search_parts_of(int clusters_cap) { return clusters_cap < 8192 ? 4 : clusters_cap < 16384 ? 2 : 1; }
 
-// Tiles of a system's pair list: pairs inside the cutoff at the mean density, 30 to
-// a tile of 64 lanes.
-static double pair_tiles_estimate(const SysDev& d) {
-  const double rho = d.n_atoms / (d.L[0] * d.L[1] * d.L[2]);
-  return 0.5 * d.n_atoms * (4.0 / 3.0 * kPi * d.rc2 * d.rc * rho) / 30.0;
-}
-
 // Tiles per pair-kernel work item, from the system alone (a system's sums must not
 // depend on the batch around it).  A wave runs an item's tiles one after the other,
 // so a list of few items is as slow as one item: 1,000 atoms (6,000 tiles) 15.2 us
@@ -575,15 +582,15 @@ static size_t items_cap(size_t groups, int clusters_cap) {
 }
 
 // Device bytes of one neighbour block (the allocations of alloc_neighbor_block).
-size_t nb_bytes(int ncol, int nzb, int mixed, long long pairs_cap, int clusters_cap) {
+size_t nb_bytes(int ncol, int nzb, bool entries, long long pairs_cap, int clusters_cap) {
   const size_t ns = (size_t)clusters_cap * CLUSTER, cc = clusters_cap;
   const size_t parts = search_parts_of(clusters_cap);
   size_t b = 2 * rnd256(4 * CNT_LINE * (size_t)ncol) + rnd256(4 * ((size_t)ncol + 1)) + 2 * rnd256(4 * (size_t)ncol * (nzb + 1));
-  (void)mixed;  // slot records have one size
   b += rnd256(4 * ns) + rnd256(ns * SLOT_BYTES) + rnd256(4 * ns) + rnd256(ns * SLOT_BYTES) +
        rnd256(4 * ns) + rnd256(4 * cc) + rnd256(32 * cc) + rnd256(24 * ns);
   b += rnd256(4 * (cc * parts + 1)) + rnd256(4 * cc * parts * SEARCH_TMP_CAP) + rnd256(8 * cc * parts * SEARCH_TMP_CAP);
   b += rnd256(4 * CNT_LINE * ((cc + 63) / 64));
+  if (entries) return b + 2 * rnd256(8 * (size_t)pairs_cap) + rnd256(8);
   const size_t gc = groups_cap(pairs_cap, clusters_cap);
   b += rnd256(16 * (gc + 1)) + rnd256(32 * (gc + 2)) + rnd256(16 * items_cap(gc, clusters_cap)) + rnd256(8);
   return b;
@@ -643,13 +650,19 @@ int System::alloc_neighbor_block(long long pairs_cap, int clusters_cap) {
   FZ_TRY(dalloc(&d.search_tmp, (size_t)clusters_cap * d.search_parts * SEARCH_TMP_CAP, false));
   FZ_TRY(dalloc(&d.search_mtmp, (size_t)clusters_cap * d.search_parts * SEARCH_TMP_CAP, false));
   FZ_TRY(dalloc(&d.tile_cnt, CNT_LINE * (((size_t)clusters_cap + 63) / 64)));
+  if (d.entry_list) {
+    FZ_TRY(dalloc(&d.pl_ij, pairs_cap, false));
+    FZ_TRY(dalloc(&d.pl_mask, pairs_cap, false));
+    FZ_TRY(dalloc(&d.pg_n, 1));
+    return FZ_OK;
+  }
   d.n_groups_cap = (long long)groups_cap(pairs_cap, clusters_cap);
   // the pair kernel reads one mask and two groups of offsets ahead
   FZ_TRY(dalloc(&d.pg_mask, (size_t)d.n_groups_cap + 1, false));
   FZ_TRY(dalloc(&d.pg_j, ((size_t)d.n_groups_cap + 2) * 8, false));
   FZ_TRY(dalloc(&d.pg_item, items_cap((size_t)d.n_groups_cap, clusters_cap), false));
   FZ_TRY(dalloc(&d.pg_n, 1));
-  d.item_tiles = pair_item_tiles(pair_tiles_estimate(d));
+  d.item_tiles = pair_item_tiles(pair_tiles_estimate(d.n_atoms, d.L, d.rc));
   return FZ_OK;
 }
 
@@ -692,7 +705,7 @@ int64_t footprint_bytes(const fz_topology* t, const fz_params* p, int precision)
     pairs = (long long)(pairs * 1.6) + 4096;
     clus = (int)(clus * 1.3) + 64;
   }
-  b += nb_bytes(sh.ncol, sh.nzb, mixed, pairs, clus);
+  b += nb_bytes(sh.ncol, sh.nzb, has_entry_list(mixed, pair_tiles_estimate(t->n_atoms, p->box, p->cutoff)) != 0, pairs, clus);
   return (int64_t)b;
 }
 
@@ -973,8 +986,8 @@ int Engine::prepare() {
   if (!status_) FZ_HIP(hipHostMalloc((void**)&status_, ns * sizeof(StatusRec), hipHostMallocDefault));
   for (int** cp : {&L_.chunk_pre, &L_.chunk_pre_a}) {
     if (*cp) continue;
-    FZ_HIP(hipMalloc(cp, (ns + 1) * sizeof(int)));
-    FZ_HIP(hipMemset(*cp, 0, (ns + 1) * sizeof(int)));
+    FZ_HIP(hipMalloc(cp, 2 * (ns + 1) * sizeof(int)));
+    FZ_HIP(hipMemset(*cp, 0, 2 * (ns + 1) * sizeof(int)));
   }
   FZ_TRY(upload_desc());
   L_.d_sys = d_sys_;
@@ -1049,15 +1062,22 @@ int Engine::prepare() {
   // takes 491-500 us with 4,096 blocks and 472 with 16,384, of 131,000 in FP64 517-534
   // and 518-522, of 19,000 98-100 us with 1,152 and 96-97 with 2,048.
   long long atoms_total = 0;
-  double items4 = 0.0;
+  double items4 = 0.0, chunks = 0.0;
+  L_.n_entry = 0;
   for (auto* s : sys_) {
     const SysDev& d = s->dv;
     atoms_total += d.n_atoms;
-    const double t = pair_tiles_estimate(d);
-    items4 += 1.3 * t / (4.0 * pair_item_tiles(t));  // items are cut per pair of clusters: some are short
+    const double t = pair_tiles_estimate(d.n_atoms, d.L, d.rc);
+    if (d.entry_list) {
+      L_.n_entry++;
+      chunks += 1.6 * t / PAIR_CHUNK;  // a tile of two whole clusters has fewer pairs
+    } else {
+      items4 += 1.3 * t / (4.0 * pair_item_tiles(t));  // items are cut per pair of clusters: some are short
+    }
   }
   const int grid0 = items4 >= 16384.0 ? 16384 : std::max(256, ((int)items4 + 63) / 64 * 64);
   L_.pair_grid = tuned_grid_ > 0 ? tuned_grid_ : grid0;
+  L_.entry_grid = tuned_grid_ > 0 ? tuned_grid_ : chunks >= 8192.0 ? 8192 : std::max(64, (int)chunks);
   // Spread by bricks from 24K atoms per launch; below, the single atomic kernel is
   // cheaper than the brick pipeline's four launches.  Same grid either way.  Steps,
   // atomics -> bricks: 17,000 atoms 102 -> 105 us, 21,000 113 -> 114, 42,000 161 -> 138,

@@ -213,7 +213,7 @@ struct NbShape {
 };
 NbShape nb_shape(const fz_params& par, int n, int ncx, int ncy, double f);
 // device bytes of one neighbour block
-size_t nb_bytes(int ncol, int nzb, int mixed, long long pairs_cap, int clusters_cap);
+size_t nb_bytes(int ncol, int nzb, bool entries, long long pairs_cap, int clusters_cap);
 // upper bound of one system's device bytes (the serving admission figure)
 int64_t footprint_bytes(const fz_topology* t, const fz_params* p, int precision);
 

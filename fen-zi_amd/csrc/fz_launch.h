@@ -75,9 +75,11 @@ struct Launch {
   Work w_fftz;    // z-line groups
   Work w_bricks;  // one block per PME brick
   Work w_planes;  // one block per PME grid z plane
-  int* chunk_pre = nullptr;  // device: pair-kernel work items per system (prefix; a single system's are in its pg_n)
+  int* chunk_pre = nullptr;  // device: pair-kernel work items per system (prefix; a single system's are in its pg_n), then those of entry lists
   int* chunk_pre_a = nullptr;  // device: the same for the systems without a pending rebuild
   int pair_grid = 0;         // persistent pair-kernel blocks
+  int n_entry = 0;           // systems with an entry list (a kernel of their own)
+  int entry_grid = 0;        // its blocks
   int fft_lds = 0;           // dynamic LDS bytes for the FFT kernels
   int fft_nl = 16;           // lines per FFT workgroup
   int lj_sep = 0;            // every system follows the LJ combination rule

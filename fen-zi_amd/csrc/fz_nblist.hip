@@ -854,6 +854,39 @@ __device__ __forceinline__ void fill_scan(const SysDev& d, const FillList (&l)[2
   }
 }
 
+// The entries of the clusters I0 and I0 + 1 of an entry list into place: offset, the
+// counts of the 64-cluster tiles before theirs and of the clusters before I0 inside it.
+__device__ __forceinline__ void fill_entries(const SysDev& d, int I0, int n, int split) {
+  const int lane = threadIdx.x & 63;
+  if (I0 >= n) return;
+  const FillList l[2] = {fill_list(d, I0, true, split), fill_list(d, I0 + 1, I0 + 1 < n, split)};
+  const int t = I0 >> 6, nt = (n + 63) >> 6;
+  long long before = 0, total = 0;
+  for (int k = lane; k < nt; k += 64) {
+    const long long v = d.tile_cnt[CNT_LINE * k];
+    total += v;
+    if (k < t) before += v;
+  }
+  for (int k = (t << 6) * split + lane; k < I0 * split; k += 64) before += d.search_cnt[k];
+  before = wave_sum(before);
+  total = wave_sum(total);
+  if (I0 == 0 && lane == 0) {
+    if (total > d.n_pairs_cap) atomicOr(d.flags + F_OVERFLOW, OV_PAIRS);
+    else d.flags[F_NBUILD] += 1;
+    *d.n_pairs = total > d.n_pairs_cap ? 0 : total;
+  }
+  if (total > d.n_pairs_cap) return;
+  const int n0 = l[0].total, n01 = n0 + l[1].total;
+#pragma unroll 4
+  for (int k = lane; k < n01; k += 64) {
+    const size_t at = k < n0 ? l[0].at(k) : l[1].at(k - n0);
+    const int J = d.search_tmp[at];
+    const unsigned long long m = d.search_mtmp[at];
+    d.pl_ij[before + k] = make_int2(k < n0 ? I0 : I0 + 1, J);
+    d.pl_mask[before + k] = m;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S, int nsys, const int* __restrict__ pre,
                                                    int split_cap) {
   SYS_FROM(pre);
@@ -867,6 +900,10 @@ __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S,
   if (2 * (lb * 4) >= n) return;  // the whole block
   const bool live = I0 < n, two = I0 + 1 < n;
   const int split = search_split(d.search_parts, split_cap);
+  if (d.entry_list) {
+    fill_entries(d, I0, n, split);
+    return;
+  }
   const FillList l[2] = {fill_list(d, I0, live, split), fill_list(d, I0 + 1, two, split)};
   long long total = 0;
   for (int k = threadIdx.x; k < (n + 63) >> 6; k += 256) total += d.tile_cnt[CNT_LINE * k];

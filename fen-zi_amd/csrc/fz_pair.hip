@@ -46,8 +46,12 @@ __global__ __launch_bounds__(256) void k_gather_sorted(const SysDev* __restrict_
   store_slot(d, sl, d.slot_atom[sl]);
 }
 
-// One block: the pair kernel's work items (none of a system after an overflow)
-// as a prefix over the systems of a batch.
+// chunks of an entry list
+__device__ __forceinline__ int entry_chunks(const SysDev& d) { return (int)((*d.n_pairs + PAIR_CHUNK - 1) / PAIR_CHUNK); }
+
+// One block: the pair kernels' work items (none of a system after an overflow)
+// as prefixes over the systems of a batch: those of pair groups, then those of
+// entry lists (low and high word of one scan).
 // Systems are taken 1024 at a time, one per thread, with a block scan and a
 // running carry.  MODE 0: every system, and the rebuild decisions are spent;
 // MODE 1: only the systems without a pending rebuild (their lists are valid
@@ -55,28 +59,34 @@ __global__ __launch_bounds__(256) void k_gather_sorted(const SysDev* __restrict_
 // and the rebuild decisions are spent.
 template <int MODE>
 __global__ __launch_bounds__(1024) void k_chunk_prefix(const SysDev* __restrict__ S, int nsys, int* __restrict__ chunk_pre) {
-  __shared__ int part[1024];
-  __shared__ int carry;
+  __shared__ unsigned long long part[1024];
+  __shared__ unsigned long long carry;
   const int t = threadIdx.x;
-  if (t == 0) { carry = 0; chunk_pre[0] = 0; }
+  int* entry_pre = chunk_pre + nsys + 1;
+  if (t == 0) { carry = 0ull; chunk_pre[0] = entry_pre[0] = 0; }
   for (int base = 0; base < nsys; base += 1024) {
     const int s = base + t;
-    int c = 0;
+    unsigned long long c = 0ull;
     if (s < nsys) {
       const bool pending = S[s].flags[F_REBUILD] != 0;
       const bool take = MODE == 0 || (MODE == 1 ? !pending : pending);
-      c = (S[s].flags[F_OVERFLOW] || !take) ? 0 : (int)(*S[s].pg_n >> 40);
+      if (take && !S[s].flags[F_OVERFLOW])
+        c = S[s].entry_list ? (unsigned long long)(unsigned)entry_chunks(S[s]) << 32 : *S[s].pg_n >> 40;
       if (MODE != 1) S[s].flags[F_REBUILD] = 0;
     }
     part[t] = c;
     __syncthreads();
     for (int o = 1; o < 1024; o <<= 1) {  // Hillis-Steele inclusive scan
-      const int v = t >= o ? part[t - o] : 0;
+      const unsigned long long v = t >= o ? part[t - o] : 0ull;
       __syncthreads();
       part[t] += v;
       __syncthreads();
     }
-    if (s < nsys) chunk_pre[s + 1] = carry + part[t];
+    if (s < nsys) {
+      const unsigned long long v = carry + part[t];
+      chunk_pre[s + 1] = (int)(unsigned)v;
+      entry_pre[s + 1] = (int)(unsigned)(v >> 32);
+    }
     __syncthreads();
     if (t == 1023) carry += part[1023];
     __syncthreads();
@@ -140,6 +150,9 @@ typedef FZ_GLOBAL v2f GF2;
 // work items and group masks are read through the scalar cache: the address is
 // the wave's, and a scalar load leaves the vector memory counter to the j gathers
 typedef const __attribute__((address_space(4))) v4i CI4;
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef const __attribute__((address_space(4))) v2i CI2;
+typedef const __attribute__((address_space(4))) unsigned long long CU64;
 typedef FZ_GLOBAL unsigned long long GU64;
 
 __device__ __forceinline__ void atomic_add_g(GU64* p, unsigned long long v) {
@@ -299,7 +312,13 @@ struct ICluster {
   int x, y, z, t;      // position top words, LJ table row
   float q, q_raw;      // charge times the Coulomb constant, charge
   v2f p;               // LJ parameters
-  float fx, fy, fz;    // force sums
+  __device__ __forceinline__ void set(const v4i& v, const v2f& lp, int n_types) {
+    p = lp;
+    x = v.x; y = v.y; z = v.z;
+    q_raw = __int_as_float(v.w);
+    q = q_raw * (float)CC;
+    t = __float_as_int(lp.x) * n_types;
+  }
 };
 
 // Horner's rule over one of the Ewald polynomials.  The coefficients are scalars of
@@ -352,13 +371,19 @@ __device__ __forceinline__ float add_rn(float a, float b) {
 #pragma clang fp contract(off)
   return a + b;
 }
+__device__ __forceinline__ void sub3_rn(float (&f)[3], float x, float y, float z) {
+  f[0] = add_rn(f[0], -x);
+  f[1] = add_rn(f[1], -y);
+  f[2] = add_rn(f[2], -z);
+}
 
 // One tile: forces of the lane's pair on its j (fx, fy, fz), energies into cev;
 // returns the lanes with a pair inside the cutoff.
 template <int EV, bool SEP>
 __device__ __forceinline__ unsigned long long tile_mixed(const SysDev& d, const PairConst& c, const GF2* lj,
-                                                         unsigned long long mask, ICluster& ic, const v4i& xj, const v2f& pj,
-                                                         float& fx, float& fy, float& fz, double (&cev)[8], int& npr) {
+                                                         unsigned long long mask, const ICluster& ic, const v4i& xj,
+                                                         const v2f& pj, float& fx, float& fy, float& fz, double (&cev)[8],
+                                                         int& npr) {
   const float dx = (float)(int)((unsigned)xj.x - (unsigned)ic.x) * c.sx;
   const float dy = (float)(int)((unsigned)xj.y - (unsigned)ic.y) * c.sy;
   const float dz = (float)(int)((unsigned)xj.z - (unsigned)ic.z) * c.sz;
@@ -409,7 +434,6 @@ __device__ __forceinline__ unsigned long long tile_mixed(const SysDev& d, const 
   // F / r = (r2 F_C / r + 6 S f6) / r2 + E_LJ (-2 dS/dr2)
   const float fs = act ? fmaf(e6, dsw, fmaf(f6, sw6, fc2) * rinv2) : 0.0f;
   fx = fs * dx; fy = fs * dy; fz = fs * dz;
-  ic.fx = add_rn(ic.fx, -fx); ic.fy = add_rn(ic.fy, -fy); ic.fz = add_rn(ic.fz, -fz);
   if (EV && act) {
     if (EV == 1) {
       cev[0] += (double)(e6 * sw6 * (1.0f / 6.0f));
@@ -482,16 +506,12 @@ __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S
     const unsigned jlo = (unsigned)jl * 4u;
     unsigned jon = buf_ld1(jr, jlo, 0u), jonn = buf_ld1(jr, jlo, 32u);
     ICluster ic[2];
+    float fi[2][3] = {{0.f, 0.f, 0.f}, {0.f, 0.f, 0.f}};  // their force sums
 #pragma unroll
     for (int h = 0; h < 2; h++) {
       const unsigned so = (unsigned)(h ? I1 : I0) * (CLUSTER * SLOT_BYTES);
       const v4i v = buf_ld4(xsr, (unsigned)il * SLOT_BYTES, so);
-      ic[h].p = buf_ld2(xsr, (unsigned)il * SLOT_BYTES + 16u, so);
-      ic[h].x = v.x; ic[h].y = v.y; ic[h].z = v.z;
-      ic[h].q_raw = __int_as_float(v.w);
-      ic[h].q = ic[h].q_raw * (float)CC;
-      ic[h].t = __float_as_int(ic[h].p.x) * d.n_types;
-      ic[h].fx = ic[h].fy = ic[h].fz = 0.f;
+      ic[h].set(v, buf_ld2(xsr, (unsigned)il * SLOT_BYTES + 16u, so), d.n_types);
     }
     v4i xjn = buf_ld4(xsr, jon, 0u);
     v2f pjn = buf_ld2(xsr, jon + 16u, 0u);
@@ -515,10 +535,14 @@ __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S
       if (__builtin_amdgcn_inverse_ballot_w64(pend_m)) atomic_add_g((GU64*)(Fb + pend_o), pend_v);
       float jx = 0.f, jy = 0.f, jz = 0.f;
       unsigned long long actm = 0ull;
-      if (m0) actm = tile_mixed<EV, SEP>(d, pc, lj, m0, ic[0], xj, pj, jx, jy, jz, cev, ev.npr);
+      if (m0) {
+        actm = tile_mixed<EV, SEP>(d, pc, lj, m0, ic[0], xj, pj, jx, jy, jz, cev, ev.npr);
+        sub3_rn(fi[0], jx, jy, jz);
+      }
       if (m1) {
         float fx, fy, fz;
         actm |= tile_mixed<EV, SEP>(d, pc, lj, m1, ic[1], xj, pj, fx, fy, fz, cev, ev.npr);
+        sub3_rn(fi[1], fx, fy, fz);
         jx = add_rn(jx, fx); jy = add_rn(jy, fy); jz = add_rn(jz, fz);
       }
       // j sums: every lane of group j = lane >> 3 holds slot j's; lane 8j + c adds
@@ -530,8 +554,118 @@ __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S
       pend_o = jo + coff;
     }
     if (__builtin_amdgcn_inverse_ballot_w64(pend_m)) atomic_add_g((GU64*)(Fb + pend_o), pend_v);
-    flush_i(Fb, I0, lane, ic[0].fx, ic[0].fy, ic[0].fz);
-    if (I1 != I0) flush_i(Fb, I1, lane, ic[1].fx, ic[1].fy, ic[1].fz);
+    flush_i(Fb, I0, lane, fi[0][0], fi[0][1], fi[0][2]);
+    if (I1 != I0) flush_i(Fb, I1, lane, fi[1][0], fi[1][1], fi[1][2]);
+    if (EV) ev.add_item(cev, lane);
+  }
+  if (EV && evs >= 0) ev.flush(S[evs], lane);
+}
+
+// Mixed form over entry lists (SysDev::entry_list): tiles of two whole clusters.
+//
+// Forces on i are FP32 sums over an i cluster's run of entries within a chunk of
+// PAIR_CHUNK, in list order.  A small system's trajectory runs many steps between two
+// looks at it and multiplies a rounding difference about eightfold in 40 steps of 2 fs,
+// so the order of these sums is part of its results: it is the list's, whatever wave
+// forms a tile.  One workgroup per chunk: its four waves form the tiles of eight
+// entries each, all their records loaded before the first is used, and leave the i
+// terms in LDS; then one wave per component adds them up entry by entry.
+//
+// What bounds it: latency (1,000 atoms: 280 chunks).  A wave per chunk, as one would
+// run them with more of them than the chip has waves, took 15.2 us at 1,000 atoms.
+constexpr int ENTRY_WAVE = PAIR_CHUNK / 4;  // entries of a wave
+
+template <int EV, bool SEP>
+__global__ __launch_bounds__(256) void k_pair_entry(const SysDev* __restrict__ S, int nsys, const int* __restrict__ chunk_pre,
+                                                    int spend) {
+  if (spend && blockIdx.x == 0 && threadIdx.x == 0) S[0].flags[F_REBUILD] = 0;
+  __shared__ float term[PAIR_CHUNK][3][64];
+  const int lane = threadIdx.x & 63, il = lane & 7, jl = lane >> 3, wv = rfl(threadIdx.x >> 6);
+  chunk_pre += nsys + 1;  // the entry lists' prefix
+  const int total = rfl(nsys > 1 ? chunk_pre[nsys] : S[0].flags[F_OVERFLOW] ? 0 : entry_chunks(S[0]));
+  int evs = -1;
+  EvAcc ev;
+  ev.zero();
+  for (int w = blockIdx.x; w < total; w += gridDim.x) {
+    const int s = nsys == 1 ? 0 : rfl(locate(chunk_pre, nsys, w));
+    const int wk = nsys == 1 ? w : w - chunk_pre[s];
+    const SysDev& d = S[s];
+    if (EV && s != evs) {
+      if (evs >= 0) ev.flush(S[evs], lane);
+      ev.zero();
+      evs = s;
+    }
+    double cev[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const long long np = *d.n_pairs, e0 = (long long)wk * PAIR_CHUNK;
+    const int ne = rfl((int)(np - e0 < PAIR_CHUNK ? np - e0 : PAIR_CHUNK));
+    if (EV && wk == 0 && wv == 0) ev.ntl += np;
+    const __amdgpu_buffer_rsrc_t xsr = raw_rsrc(d.xs, (unsigned)d.n_slots_cap * SLOT_BYTES);
+    const CI2* ent = (const CI2*)(d.pl_ij + e0);
+    const CU64* msk = (const CU64*)(d.pl_mask + e0);
+    const GF2* lj = (const GF2*)d.lj32;
+    FZ_GLOBAL char* Fb = (FZ_GLOBAL char*)d.Fs;
+    const PairConst pc(d);
+    // the wave's entries (past the list's end: the last one, no lanes)
+    unsigned Js[ENTRY_WAVE];
+    unsigned long long m[ENTRY_WAVE];
+    v4i xi[ENTRY_WAVE], xj[ENTRY_WAVE];
+    v2f pi[ENTRY_WAVE], pj[ENTRY_WAVE];
+#pragma unroll
+    for (int k = 0; k < ENTRY_WAVE; k++) {
+      const int e = wv * ENTRY_WAVE + k, at = e < ne ? e : ne - 1;
+      const v2i ij = ent[at];
+      m[k] = e < ne ? msk[at] : 0ull;
+      const unsigned Is = (unsigned)ij.x * (CLUSTER * SLOT_BYTES);
+      Js[k] = (unsigned)ij.y * (CLUSTER * SLOT_BYTES);
+      xi[k] = buf_ld4(xsr, (unsigned)il * SLOT_BYTES, Is);
+      pi[k] = buf_ld2(xsr, (unsigned)il * SLOT_BYTES + 16u, Is);
+      xj[k] = buf_ld4(xsr, (unsigned)jl * SLOT_BYTES, Js[k]);
+      pj[k] = buf_ld2(xsr, (unsigned)jl * SLOT_BYTES + 16u, Js[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < ENTRY_WAVE; k++) {
+      float fx = 0.f, fy = 0.f, fz = 0.f;
+      float* t = &term[wv * ENTRY_WAVE + k][0][lane];
+      unsigned long long actm = 0ull;
+      if (m[k]) {
+        ICluster ic;
+        ic.set(xi[k], pi[k], d.n_types);
+        actm = tile_mixed<EV, SEP>(d, pc, lj, m[k], ic, xj[k], pj[k], fx, fy, fz, cev, ev.npr);
+      }
+      t[0] = fx; t[64] = fy; t[128] = fz;
+      if (m[k]) {
+        red8x3(fx, fy, fz);
+        const int c = lane & 7;
+        const unsigned long long v = fixed_f32(c == 0 ? fx : (c == 1 ? fy : fz));
+        if (__builtin_amdgcn_inverse_ballot_w64(byte_any3(actm)))
+          atomic_add_g((GU64*)(Fb + (size_t)Js[k] + (unsigned)jl * SLOT_BYTES + (unsigned)c * 8u), v);
+      }
+    }
+    __syncthreads();
+    if (wv < 3) {  // component wv of the i forces
+      float f = 0.f;
+      int I = ent[0].x;
+      auto flush = [&]() {
+        const float r = red_stride8(f);
+        if (lane < 8)
+          atomic_add_g((GU64*)(Fb + (size_t)I * (CLUSTER * SLOT_BYTES) + (unsigned)lane * SLOT_BYTES + (unsigned)wv * 8u), fixed_f32(r));
+      };
+      float t[PAIR_CHUNK];
+#pragma unroll
+      for (int k = 0; k < PAIR_CHUNK; k++) t[k] = term[k][wv][lane];
+#pragma unroll
+      for (int k = 0; k < PAIR_CHUNK; k++) {
+        const int Ik = k < ne ? ent[k].x : I;
+        if (Ik != I) {
+          flush();
+          f = 0.f;
+          I = Ik;
+        }
+        f = add_rn(f, -t[k]);
+      }
+      flush();
+    }
+    __syncthreads();
     if (EV) ev.add_item(cev, lane);
   }
   if (EV && evs >= 0) ev.flush(S[evs], lane);
@@ -665,31 +799,43 @@ __global__ __launch_bounds__(256) void k_pair_f64(const SysDev* __restrict__ S, 
   if (EV && evs >= 0) ev.flush(S[evs], lane);
 }
 
+template <int EV, bool SEP>
+static void launch_pair_mixed(const Launch& L, const int* cp, int sp) {
+  if (L.n_entry < L.nsys)
+    hipLaunchKernelGGL((k_pair_mixed<EV, SEP>), dim3(L.pair_grid), dim3(256), 0, L.stream, L.d_sys, L.nsys, cp, sp);
+  if (L.n_entry > 0)
+    hipLaunchKernelGGL((k_pair_entry<EV, SEP>), dim3(L.entry_grid), dim3(256), 0, L.stream, L.d_sys, L.nsys, cp, sp);
+}
+
+template <bool EV, bool POLY>
+static void launch_pair_f64(const Launch& L, const int* cp, int sp) {
+  hipLaunchKernelGGL((k_pair_f64<EV, POLY>), dim3(L.pair_grid), dim3(256), 0, L.stream, L.d_sys, L.nsys, cp, sp);
+}
+
 void launch_pair(const Launch& L, int ev, const int* cp, bool fold, bool spend) {
   const int sp = spend ? 1 : 0;
-  dim3 g(L.pair_grid), b(256);
   if (!cp) cp = L.chunk_pre;
   if (L.mixed) {
     if (ev == 2 && !L.ew_poly) ev = 3;
     if (L.lj_sep) {
-      if (ev == 3) hipLaunchKernelGGL((k_pair_mixed<3, true>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else if (ev == 2) hipLaunchKernelGGL((k_pair_mixed<2, true>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else if (ev == 1) hipLaunchKernelGGL((k_pair_mixed<1, true>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else hipLaunchKernelGGL((k_pair_mixed<0, true>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
+      if (ev == 3) launch_pair_mixed<3, true>(L, cp, sp);
+      else if (ev == 2) launch_pair_mixed<2, true>(L, cp, sp);
+      else if (ev == 1) launch_pair_mixed<1, true>(L, cp, sp);
+      else launch_pair_mixed<0, true>(L, cp, sp);
     } else {
-      if (ev == 3) hipLaunchKernelGGL((k_pair_mixed<3, false>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else if (ev == 2) hipLaunchKernelGGL((k_pair_mixed<2, false>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else if (ev == 1) hipLaunchKernelGGL((k_pair_mixed<1, false>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else hipLaunchKernelGGL((k_pair_mixed<0, false>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
+      if (ev == 3) launch_pair_mixed<3, false>(L, cp, sp);
+      else if (ev == 2) launch_pair_mixed<2, false>(L, cp, sp);
+      else if (ev == 1) launch_pair_mixed<1, false>(L, cp, sp);
+      else launch_pair_mixed<0, false>(L, cp, sp);
     }
   } else {
     // the Ewald polynomials wherever every system has them
     if (L.ew_poly) {
-      if (ev) hipLaunchKernelGGL((k_pair_f64<true, true>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else hipLaunchKernelGGL((k_pair_f64<false, true>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
+      if (ev) launch_pair_f64<true, true>(L, cp, sp);
+      else launch_pair_f64<false, true>(L, cp, sp);
     } else {
-      if (ev) hipLaunchKernelGGL((k_pair_f64<true, false>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
-      else hipLaunchKernelGGL((k_pair_f64<false, false>), g, b, 0, L.stream, L.d_sys, L.nsys, cp, sp);
+      if (ev) launch_pair_f64<true, false>(L, cp, sp);
+      else launch_pair_f64<false, false>(L, cp, sp);
     }
   }
   if (ev && fold) launch_ev_fold(L);

@@ -9,6 +9,7 @@
 namespace fz {
 
 constexpr int CLUSTER = 8;          // atoms per cluster (8 x 8 pair tile = one wave64)
+constexpr int PAIR_CHUNK = 32;      // entries per pair-kernel work item of an entry list
 constexpr int MIN_ITEM_TILES = 8;    // fewest tiles per pair-kernel work item (SysDev::item_tiles)
 constexpr int SLOT_BYTES = 32;      // one slot record of xs, and one slot of Fs (x, y, z, unused)
 // Counters that many blocks add to lie one to a 64-byte line (this many ints): atomics
@@ -160,6 +161,11 @@ struct SysDev {
   int4 *pg_item;         // work items: first group, groups, clusters 2 s and 2 s + 1
   unsigned long long *pg_n;  // device scalar: groups in use (low 40 bits), work items (high 24)
   int item_tiles;        // tiles per work item (pair_item_tiles)
+  // Small systems in the mixed form have no groups but the entries in list order
+  // (k_pair_entry), work items of PAIR_CHUNK.
+  int entry_list;
+  int2 *pl_ij;                  // [n_pairs_cap] clusters I, J
+  unsigned long long *pl_mask;  // [n_pairs_cap] lane masks: lane 8 j + i
   // ---- exclusions ---------------------------------------------------------
   unsigned long long *excl_bits; // [n_atoms]: bit (32 + j - i) set if j excluded, |j-i| <= 31
   int *excl_off, *excl_list;     // CSR (used when use_excl_list)
