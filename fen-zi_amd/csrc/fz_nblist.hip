@@ -46,6 +46,16 @@ __global__ __launch_bounds__(256) void k_check(const SysDev* __restrict__ S, int
 __device__ __forceinline__ bool skip_build(const SysDev& d) {
   return d.flags[F_REBUILD] == 0 || d.flags[F_OVERFLOW] != 0;
 }
+// The same answer for every wave of the block.  The pair search and the fill raise
+// F_OVERFLOW themselves: waves that each read it would leave one by one, and those
+// left behind pass the barriers (an ended wave no longer counts) without the words in
+// LDS that the others owe them.
+__device__ __forceinline__ bool skip_build_block(const SysDev& d) {
+  __shared__ int skip;
+  if (threadIdx.x == 0) skip = skip_build(d);
+  __syncthreads();
+  return skip != 0;
+}
 
 // Last block done: each of the system's nblocks blocks takes a ticket once its
 // device-scope atomics are performed; the block that draws the last ticket sees every
@@ -454,7 +464,7 @@ constexpr int HIT_RING = 128;
 __global__ __launch_bounds__(256, 5) void k_pair_search(
     const SysDev* __restrict__ S, int nsys, const int* __restrict__ pre, int split_cap) {
   SYS_FROM(pre);
-  if (skip_build(d)) return;
+  if (skip_build_block(d)) return;
   __shared__ int block_cnt[2];  // entries, waves done
   if (threadIdx.x == 0) block_cnt[0] = block_cnt[1] = 0;
   __syncthreads();
@@ -890,7 +900,7 @@ __device__ __forceinline__ void fill_entries(const SysDev& d, int I0, int n, int
 __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S, int nsys, const int* __restrict__ pre,
                                                    int split_cap) {
   SYS_FROM(pre);
-  if (skip_build(d)) return;
+  if (skip_build_block(d)) return;
   __shared__ int4 keys[4][FILL_HASH / 4];
   __shared__ unsigned long long vals[4][FILL_HASH];
   __shared__ unsigned long long need[4];  // groups (low 40 bits) and items of each wave, then their offsets
