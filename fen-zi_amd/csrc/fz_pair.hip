@@ -42,7 +42,8 @@ __global__ __launch_bounds__(256) void k_gather_sorted(const SysDev* __restrict_
   const int s_ = block_sys(pre, nsys, blockIdx.x);
   const SysDev& d = S[s_];
   const int sl = (blockIdx.x - block_base(pre, nsys, s_)) * 256 + threadIdx.x;
-  if (sl >= *d.n_clusters * CLUSTER) return;
+  // (more clusters than the capacity: counted by a build that was then left out)
+  if (sl >= min(*d.n_clusters * CLUSTER, d.n_slots_cap)) return;
   store_slot(d, sl, d.slot_atom[sl]);
 }
 

@@ -41,7 +41,8 @@ template <bool MIXED>
 __global__ __launch_bounds__(256) void k_com_force(const SysDev* __restrict__ S, int nsys, const int* __restrict__ pre) {
   const int s_ = block_sys(pre, nsys, blockIdx.x);
   const SysDev& d = S[s_];
-  if (!d.com_on) return;
+  // (a build left out for want of clusters has placed no atom in the slots there are now)
+  if (!d.com_on || d.flags[F_OVERFLOW]) return;
   const int i = (blockIdx.x - block_base(pre, nsys, s_)) * 256 + threadIdx.x;
   if (i >= d.n_atoms || d.com_grp[i] != 1) return;
   double dr[3];
