@@ -6,9 +6,10 @@
 // law instead of a full list.
 //
 // One wave64 evaluates one or two 8x8 tiles (an i cluster x eight j slots) per
-// pair group: lane l holds i = l & 7, j = l >> 3.  j forces are summed over the
-// group's tiles and the 8 lanes that share j (xor 1, 2, 4) and added once per
-// group; i forces stay in registers for the whole work item (a run of the groups
+// pair group: lane l holds i = l & 7, j = l >> 3.  j forces are summed over the 8
+// lanes that share j (xor 1, 2, 4), tile by tile, and added once per group (in the
+// mixed form the tiles' sums are added in fixed point: a sum of both in FP32 would
+// round once more and saved nothing, 227,000 atoms 288 and 290 us); i forces stay in registers for the whole work item (a run of the groups
 // of two clusters), then are reduced over lanes l, l+8, ... (xor 8, 16, 32).
 //
 // What bounds it: vector issue (every lane of a tile costs the same whether its
@@ -20,8 +21,7 @@
 // slots one by one, without those no atom of the i cluster is near: 0.48 and 0.42
 // of the lanes, a third fewer tiles.  With a list per i cluster the atomics then
 // bound the kernel (227,000 atoms: 400 us, 234 without them); two neighbouring
-// clusters share their groups, which leaves 0.64 of the cache lines and saves one
-// j reduction in three.  A j slot's record is one 32-byte sector, gathered with a
+// clusters share their groups, which leaves 0.64 of the cache lines.  A j slot's record is one 32-byte sector, gathered with a
 // per-lane byte offset that the list holds ready (no address arithmetic).
 //
 // Mixed form: int32 fixed-point displacements (the top 32 bits of the 64-bit
@@ -534,23 +534,23 @@ __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S
       pjn = buf_ld2(xsr, jon + 16u, 0u);
       jonn = buf_ld1(jr, jlo, (unsigned)(k + 2) * 32u);
       if (__builtin_amdgcn_inverse_ballot_w64(pend_m)) atomic_add_g((GU64*)(Fb + pend_o), pend_v);
-      float jx = 0.f, jy = 0.f, jz = 0.f;
-      unsigned long long actm = 0ull;
-      if (m0) {
-        actm = tile_mixed<EV, SEP>(d, pc, lj, m0, ic[0], xj, pj, jx, jy, jz, cev, ev.npr);
-        sub3_rn(fi[0], jx, jy, jz);
-      }
-      if (m1) {
-        float fx, fy, fz;
-        actm |= tile_mixed<EV, SEP>(d, pc, lj, m1, ic[1], xj, pj, fx, fy, fz, cev, ev.npr);
-        sub3_rn(fi[1], fx, fy, fz);
-        jx = add_rn(jx, fx); jy = add_rn(jy, fy); jz = add_rn(jz, fz);
-      }
       // j sums: every lane of group j = lane >> 3 holds slot j's; lane 8j + c adds
-      // component c when a pair of slot j is inside the cutoff
-      red8x3(jx, jy, jz);
-      const int c = lane & 7;
-      pend_v = fixed_f32(c == 0 ? jx : (c == 1 ? jy : jz));
+      // component c when a pair of slot j is inside the cutoff.  Each tile's sum is
+      // converted by itself and the two are added in fixed point.
+      unsigned long long actm = 0ull;
+      pend_v = 0ull;
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const unsigned long long m = h ? m1 : m0;
+        if (m) {
+          float fx, fy, fz;
+          actm |= tile_mixed<EV, SEP>(d, pc, lj, m, ic[h], xj, pj, fx, fy, fz, cev, ev.npr);
+          sub3_rn(fi[h], fx, fy, fz);
+          red8x3(fx, fy, fz);
+          const int c = lane & 7;
+          pend_v += fixed_f32(c == 0 ? fx : (c == 1 ? fy : fz));
+        }
+      }
       pend_m = byte_any3(actm);
       pend_o = jo + coff;
     }
