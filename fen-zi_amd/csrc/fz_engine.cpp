@@ -307,47 +307,46 @@ int System::init(const fz_topology* t, const fz_params* p, int precision, int de
   return alloc_device();
 }
 
-// Polynomials of the FP64 real-space Ewald terms.  With z = beta r,
-//   erfc(z) / r = 1/r - beta e(z^2),                       e(x) = erf(z) / z
-//   F_C / r     = 1/r^3 - beta^3 f(x),                     f(x) = erf(z) / z^3 - 2/sqrt(pi) e^{-x} / x
-// per unit charge product; e and f are entire functions of x,
-//   e(x) = 2/sqrt(pi) e^{-x} sum_{n>=0} (2x)^n / (2n+1)!!,  f(x) = 2/sqrt(pi) e^{-x} sum_{n>=1} 2^n x^{n-1} / (2n+1)!!,
-// so a Chebyshev interpolant in y = 2 x / X - 1 over [0, X], X = (beta rc)^2, converges
-// geometrically: with 24 points and X = 12.25 it is off by less than the rounding of
-// its evaluation (1e-16 rms).  Rewritten in powers of y: the coefficients stay below
-// 0.5, so Horner's rule in FP64 is as good.
+// Polynomial in y = (2 x - hi - lo) / (hi - lo) that interpolates f at the N Chebyshev
+// points of [lo, hi], in powers of y.
+template <int N, class F>
+static void cheb_fit(long double lo, long double hi, F&& f, double (&out)[N]) {
+  const long double pi = 3.14159265358979323846264338327950288L;
+  long double v[N], m[N] = {0.0L}, t0[N] = {1.0L}, t1[N] = {0.0L, 1.0L};
+  for (int k = 0; k < N; k++) v[k] = f(lo + (hi - lo) * 0.5L * (1.0L + cosl(pi * (2 * k + 1) / (2 * N))));
+  for (int j = 0; j < N; j++) {
+    long double c = 0.0L;
+    for (int k = 0; k < N; k++) c += v[k] * cosl(pi * j * (2 * k + 1) / (2 * N));
+    c *= (j ? 2.0L : 1.0L) / N;
+    for (int k = 0; k <= j; k++) m[k] += c * t0[k];  // t0 = T_j, t1 = T_{j+1}
+    long double t2[N];
+    for (int k = 0; k < N; k++) t2[k] = (k ? 2.0L * t1[k - 1] : 0.0L) - t0[k];
+    for (int k = 0; k < N; k++) { t0[k] = t1[k]; t1[k] = t2[k]; }
+  }
+  for (int k = 0; k < N; k++) out[k] = (double)m[k];
+}
+
+// Polynomials of the FP64 real-space Ewald terms.  With z = beta r, per unit charge
+// product,
+//   E_C = e^{-z^2} g(z) / r,  F_C / r = e^{-z^2} (g(z) + 2 z / sqrt(pi)) / r^3,  g(z) = e^{z^2} erfc z,
+// sums and products of positive factors: nothing cancels, so a term keeps its relative
+// accuracy out to the cutoff.  g falls from 1 to 0.15 over [0, 3.5] and its Chebyshev
+// interpolant with 28 points is off by less than 1e-16 of it; 2^x over [-1/2, 1/2] takes 12.
+// Errors (rms of the forces of 900 water molecules' real-space terms at beta rc = 3.06
+// to 3.5; largest of a term's F_C): 0.9e-15 to 1.0e-15 and 2.4e-15, where the library's
+// erfc and exp of a rounded z give 1.0e-15 to 1.1e-15 and 4.5e-15.  (1/r^3 less a
+// polynomial in r^2 is shorter by 17 multiply-adds, but cancels near the cutoff: 1.1e-15
+// to 9.6e-15 and 5e-10.)
 static void fit_ewald(SysDev& d) {
-  const long double z = (long double)d.beta * d.rc, X = z * z, pi = 3.14159265358979323846264338327950288L;
+  const long double beta = d.beta, z = beta * d.rc, ln2 = 0.693147180559945309417232121458176568L;
   d.ew_poly = z <= (long double)EW_MAX_Z;
-  d.ew_a = (double)(2.0L * d.beta * d.beta / X);
   if (!d.ew_poly) return;
-  long double v[2][EW_N];
-  for (int k = 0; k < EW_N; k++) {
-    const long double x = X * 0.5L * (1.0L + cosl(pi * (2 * k + 1) / (2 * EW_N)));
-    const long double c = 2.0L / sqrtl(pi) * expl(-x);
-    long double t = 1.0L, e = 1.0L, g = 2.0L / 3.0L, f = g;
-    for (int n = 1; n < 200; n++) {
-      t *= 2.0L * x / (2 * n + 1);
-      e += t;
-      g *= 2.0L * x / (2 * n + 3);
-      f += g;
-    }
-    v[0][k] = (long double)d.beta * d.beta * d.beta * c * f;
-    v[1][k] = (long double)d.beta * c * e;
-  }
-  for (int q = 0; q < 2; q++) {
-    long double m[EW_N] = {0.0L}, t0[EW_N] = {1.0L}, t1[EW_N] = {0.0L, 1.0L};
-    for (int j = 0; j < EW_N; j++) {
-      long double c = 0.0L;
-      for (int k = 0; k < EW_N; k++) c += v[q][k] * cosl(pi * j * (2 * k + 1) / (2 * EW_N));
-      c *= (j ? 2.0L : 1.0L) / EW_N;
-      for (int k = 0; k <= j; k++) m[k] += c * t0[k];  // t0 = T_j, t1 = T_{j+1}
-      long double t2[EW_N];
-      for (int k = 0; k < EW_N; k++) t2[k] = (k ? 2.0L * t1[k - 1] : 0.0L) - t0[k];
-      for (int k = 0; k < EW_N; k++) { t0[k] = t1[k]; t1[k] = t2[k]; }
-    }
-    for (int k = 0; k < EW_N; k++) (q ? d.ew_e : d.ew_f)[k] = (double)m[k];
-  }
+  d.ew_a = 2.0 / d.rc;
+  d.ew_b = (double)(beta * 1.12837916709551257389615890312154517L);
+  d.ew_c = (double)(-beta * beta / ln2);
+  cheb_fit(0.0L, z, [](long double x) { return expl(x * x) * erfcl(x); }, d.ew_g);
+  cheb_fit(-0.5L, 0.5L, [](long double x) { return exp2l(x); }, d.ew_x);
+  for (int k = 0; k < EW_X; k++) d.ew_x[k] = ldexp(d.ew_x[k], k);  // y = 2 x
 }
 
 // Tiles of a system's pair list: pairs inside the cutoff at the mean density, 30 to

@@ -322,14 +322,15 @@ struct ICluster {
   }
 };
 
-// Horner's rule over one of the Ewald polynomials.  The coefficients are scalars of
-// the launch; written out so that they are taken from scalar registers (left to
-// itself the compiler forms v_fmac, whose addend is the destination, and copies
-// every coefficient into a vector register pair first: three instructions for one).
-__device__ __forceinline__ double ewald_poly(const double (&c)[EW_N], double y) {
-  double p = c[EW_N - 1];
+// Horner's rule.  The coefficients are scalars of the launch; written out so that they
+// are taken from scalar registers (left to itself the compiler forms v_fmac, whose
+// addend is the destination, and copies every coefficient into a vector register pair
+// first: three instructions for one).
+template <int N>
+__device__ __forceinline__ double horner_s(const double (&c)[N], double y) {
+  double p = c[N - 1];
 #pragma unroll
-  for (int k = EW_N - 2; k >= 0; k--) {
+  for (int k = N - 2; k >= 0; k--) {
     double r;
     __asm__("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(p), "v"(y), "s"(c[k]));
     p = r;
@@ -337,8 +338,17 @@ __device__ __forceinline__ double ewald_poly(const double (&c)[EW_N], double y) 
   return p;
 }
 
+// Factors of the real-space Ewald terms at distance r = r2 / sqrt(r2): ex = e^{-z^2},
+// cx = e^{z^2} erfc z, z = beta r (fit_ewald)
+__device__ __forceinline__ void ewald_factors(const SysDev& d, double r2, double r, double& ex, double& cx) {
+  const double n = __builtin_rint(r2 * d.ew_c);
+  ex = __builtin_amdgcn_ldexp(horner_s(d.ew_x, fma(r2, d.ew_c, -n)), (int)n);
+  cx = horner_s(d.ew_g, fma(r, d.ew_a, -1.0));
+}
+
 // 1 / sqrt(x) in FP64: the hardware estimate (relative error e below 2^-23) and one
-// third-order step, y (1 + e/2 + 3 e^2/8), e = 1 - x y^2
+// third-order step, y (1 + e/2 + 3 e^2/8), e = 1 - x y^2.  Off by 1.3e-16 at most (rms
+// 5.5e-17), as is the quotient 1 / sqrt(x) of two rounded operations.
 __device__ __forceinline__ double rsqrt_f64(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);
@@ -440,20 +450,28 @@ __device__ __forceinline__ unsigned long long tile_mixed(const SysDev& d, const 
       cev[0] += (double)(e6 * sw6 * (1.0f / 6.0f));
       cev[1] += (double)(qex * tp * rinv);
     } else {
+#pragma clang fp contract(off)  // as in tile_f64
       // energies of an evaluation step in FP64 from the same FP32 distance, so
       // that no FP32 bias of the erfc/exp approximations sums over millions of pairs
       const double r2d = (double)r2, rid = rsqrt_f64(r2d), ri2d = rid * rid;
       const double s2d = (double)p.y * ri2d, s6d = s2d * s2d * s2d;
       const double a6d = (double)p.x * s6d;
-      double eljd = a6d * s6d - a6d;
+      double eljd = fma(a6d, s6d, -a6d);
       if (r2d > (double)c.ron2) {
         const double c1d = (double)c.rc2 - r2d, c2d = (double)c.rc2 + 2.0 * r2d - 3.0 * (double)c.ron2;
         eljd *= c1d * c1d * c2d * d.sw_inv;
       }
       cev[0] += eljd;
       const double qq = CC * (double)ic.q_raw * (double)__int_as_float(xj.w);
-      if (EV == 2) cev[1] += qq * (rid - ewald_poly(d.ew_e, fma(r2d, d.ew_a, -1.0)));
-      else cev[1] += qq * erfc(d.beta * (r2d * rid)) * rid;
+      double ec;
+      if (EV == 2) {
+        double ex, cx;
+        ewald_factors(d, r2d, r2d * rid, ex, cx);
+        ec = ex * cx;
+      } else {
+        ec = erfc(d.beta * (r2d * rid));
+      }
+      cev[1] += qq * ec * rid;
     }
     npr++;
     cev[2] += (double)(fx * dx); cev[3] += (double)(fy * dy); cev[4] += (double)(fz * dz);
@@ -678,14 +696,15 @@ struct ICluster64 {
   double q, fx, fy, fz;
 };
 
-// One FP64 tile.  POLY: real-space Ewald terms as 1/r^3 (1/r) less a polynomial
-// in r^2 (24 fused multiply-adds); otherwise (beta rc above EW_MAX_Z) with the
-// library's erfc and exp, which took most of the kernel's 250 FP64 instructions a
-// tile: force-only launch over 131,000 atoms 652 us with them.
+// One FP64 tile.  POLY: real-space Ewald terms from polynomials (fit_ewald: 41 fused
+// multiply-adds); otherwise (beta rc above EW_MAX_Z) with the library's erfc and exp,
+// which took most of the kernel's 250 FP64 instructions a tile.  Force-only launch over
+// 131,000 atoms 652 us with the library, 395 with the polynomials.
 template <bool EV, bool POLY>
 __device__ __forceinline__ void tile_f64(const SysDev& d, const double2* __restrict__ lj, unsigned long long mask,
                                          ICluster64& ic, const Slot64& xj, int tj, double& jx, double& jy, double& jz,
                                          double (&cev)[8], int& npr) {
+#pragma clang fp contract(off)  // fused where written: the variants of the kernel then agree to the bit
   const double dx = disp_f64(xj.x - ic.x, d.sc[0]), dy = disp_f64(xj.y - ic.y, d.sc[1]), dz = disp_f64(xj.z - ic.z, d.sc[2]);
   double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
   const bool act = __builtin_amdgcn_inverse_ballot_w64(mask & __builtin_amdgcn_ballot_w64(r2 < d.rc2));
@@ -696,32 +715,36 @@ __device__ __forceinline__ void tile_f64(const SysDev& d, const double2* __restr
   const double s2 = p.y * rinv2;
   const double s6 = s2 * s2 * s2;
   const double a6 = p.x * s6, a12 = a6 * s6;
-  double e_lj = a12 - a6;
-  // CHARMM switch, clamped to 1 (slope 0) below ron
-  const double r2c = fmax(r2, d.ron2), c1 = d.rc2 - r2c, c2 = d.rc2 + 2.0 * r2c - 3.0 * d.ron2;
-  const double sw = c1 * c1 * c2 * d.sw_inv;
-  const double dsw = 12.0 * c1 * (r2c - d.ron2) * d.sw_inv;
-  const double f_lj = fma((12.0 * a12 - 6.0 * a6) * rinv2, sw, e_lj * dsw);
+  double e_lj = fma(a6, s6, -a6);
+  // CHARMM switch; below ron 1 (slope 0) itself, not its formula at ron, whose last
+  // factors cancel
+  const bool sw_on = r2 > d.ron2;
+  const double c1 = d.rc2 - r2, c2 = fma(2.0, r2, d.rc2 - 3.0 * d.ron2);
+  const double sw = sw_on ? c1 * c1 * c2 * d.sw_inv : 1.0;
+  const double dsw = sw_on ? 12.0 * c1 * (r2 - d.ron2) * d.sw_inv : 0.0;
+  const double f_lj = fma(fma(12.0, a12, -6.0 * a6) * rinv2, sw, e_lj * dsw);
   e_lj *= sw;
   const double qq = ic.q * xj.q;
   double e_c = 0.0, f_c;
   if (POLY) {
-    const double y = fma(r2, d.ew_a, -1.0);
-    f_c = qq * fma(rinv, rinv2, -ewald_poly(d.ew_f, y));
-    if (EV) e_c = qq * (rinv - ewald_poly(d.ew_e, y));
+    double ex, cx;
+    const double r = r2 * rinv;
+    ewald_factors(d, r2, r, ex, cx);
+    f_c = qq * (ex * fma(r, d.ew_b, cx)) * (rinv * rinv2);
+    if (EV) e_c = qq * rinv * (ex * cx);
   } else {
     const double x = d.beta * (r2 * rinv);
     e_c = qq * erfc(x) * rinv;
-    f_c = (e_c + qq * (TWO_OVER_SQRT_PI * d.beta) * exp(-x * x)) * rinv2;
+    f_c = fma(qq * (TWO_OVER_SQRT_PI * d.beta), exp(-x * x), e_c) * rinv2;
   }
   const double fs = act ? f_c + f_lj : 0.0;
-  const double fx = fs * dx, fy = fs * dy, fz = fs * dz;
-  ic.fx -= fx; ic.fy -= fy; ic.fz -= fz;
-  jx += fx; jy += fy; jz += fz;
+  ic.fx = fma(-fs, dx, ic.fx); ic.fy = fma(-fs, dy, ic.fy); ic.fz = fma(-fs, dz, ic.fz);
+  jx = fma(fs, dx, jx); jy = fma(fs, dy, jy); jz = fma(fs, dz, jz);
   if (EV && act) {
+    const double fx = fs * dx, fy = fs * dy, fz = fs * dz;
     cev[0] += e_lj; cev[1] += e_c; npr++;
-    cev[2] += fx * dx; cev[3] += fy * dy; cev[4] += fz * dz;
-    cev[5] += fx * dy; cev[6] += fx * dz; cev[7] += fy * dz;
+    cev[2] = fma(fx, dx, cev[2]); cev[3] = fma(fy, dy, cev[3]); cev[4] = fma(fz, dz, cev[4]);
+    cev[5] = fma(fx, dy, cev[5]); cev[6] = fma(fx, dz, cev[6]); cev[7] = fma(fy, dz, cev[7]);
   }
 }
 

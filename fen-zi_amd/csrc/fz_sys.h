@@ -18,7 +18,7 @@ constexpr int CNT_LINE = 16;
 constexpr int SEARCH_TMP_CAP = 512;  // max J clusters per I cluster in the search buffer
 constexpr int MAX_COLUMN_ATOMS = 2048; // LDS sort capacity per column
 constexpr int MAX_FFT = 256;        // largest PME grid dimension
-constexpr int EW_N = 24;            // coefficients of the FP64 Ewald polynomials
+constexpr int EW_N = 28, EW_X = 12; // coefficients of the FP64 Ewald polynomials: erfc part, exponential
 constexpr double EW_MAX_Z = 3.5;    // largest beta rc they are fitted for
 
 // Energy / virial accumulator slots (int64 fixed point, scale 2^32).
@@ -100,11 +100,11 @@ struct SysDev {
   double rc2, ron2, rl2, skin2;   // cutoff^2, switch-on^2, pair-list^2, (0.5*(rl-rc))^2
   double beta;
   double sw_inv;         // 1 / (rc^2 - ron^2)^3
-  // Real-space Ewald in FP64 as polynomials in y = ew_a r^2 - 1 in [-1, 1]: ew_f for
-  // beta^3 (erf z / z^3 - 2/sqrt(pi) e^{-z^2} / z^2), ew_e for beta erf z / z, z = beta r
-  // (ew_poly: beta rc <= EW_MAX_Z; fit_ewald)
+  // Real-space Ewald in FP64 (ew_poly: beta rc <= EW_MAX_Z; fit_ewald), z = beta r:
+  // e^{-z^2} = 2^n ew_x(t - n), t = ew_c r^2, n its nearest whole number;
+  // e^{z^2} erfc z = ew_g(ew_a r - 1); ew_b = 2 beta / sqrt(pi)
   int ew_poly;
-  double ew_a, ew_f[EW_N], ew_e[EW_N];
+  double ew_a, ew_b, ew_c, ew_g[EW_N], ew_x[EW_X];
   double dt;             // AKMA time step (TU * dt_ps)
   double shake_tol;
   double pme_pre;        // CC / (pi V)
