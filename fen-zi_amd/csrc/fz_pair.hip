@@ -464,7 +464,7 @@ __device__ __forceinline__ unsigned long long tile_mixed(const SysDev& d, const 
       cev[0] += eljd;
       const double qq = CC * (double)ic.q_raw * (double)__int_as_float(xj.w);
       double ec;
-      if (EV == 2) {
+      if (EV == 2 || d.ew_poly) {
         double ex, cx;
         ewald_factors(d, r2d, r2d * rid, ex, cx);
         ec = ex * cx;
@@ -482,8 +482,8 @@ __device__ __forceinline__ unsigned long long tile_mixed(const SysDev& d, const 
 
 // EV: 0 forces only; 1 also energies and virial summed from the FP32 pair terms
 // (the minimisers' accept/reject tests); 2 energies recomputed in FP64 from the
-// FP32 distance (reported energies), 3 the same with the library's erfc (some
-// system has no Ewald polynomials).  SEP: every system of the launch follows the
+// FP32 distance (reported energies), 3 the same in a launch with a system that has
+// no Ewald polynomials (that one: the library's erfc).  SEP: every system of the launch follows the
 // combination rule (per-slot LJ parameters, no table lookup).
 template <int EV, bool SEP>
 __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S, int nsys, const int* __restrict__ chunk_pre,
@@ -696,10 +696,11 @@ struct ICluster64 {
   double q, fx, fy, fz;
 };
 
-// One FP64 tile.  POLY: real-space Ewald terms from polynomials (fit_ewald: 41 fused
-// multiply-adds); otherwise (beta rc above EW_MAX_Z) with the library's erfc and exp,
-// which took most of the kernel's 250 FP64 instructions a tile.  Force-only launch over
-// 131,000 atoms 652 us with the library, 395 with the polynomials.
+// One FP64 tile.  Real-space Ewald terms from polynomials (fit_ewald: 41 fused
+// multiply-adds); of a system without them (beta rc above EW_MAX_Z) with the library's
+// erfc and exp, which took most of the kernel's 250 FP64 instructions a tile.
+// Force-only launch over 131,000 atoms 652 us with the library, 395 with the polynomials.
+// POLY: every system of the launch has them.
 template <bool EV, bool POLY>
 __device__ __forceinline__ void tile_f64(const SysDev& d, const double2* __restrict__ lj, unsigned long long mask,
                                          ICluster64& ic, const Slot64& xj, int tj, double& jx, double& jy, double& jz,
@@ -726,7 +727,7 @@ __device__ __forceinline__ void tile_f64(const SysDev& d, const double2* __restr
   e_lj *= sw;
   const double qq = ic.q * xj.q;
   double e_c = 0.0, f_c;
-  if (POLY) {
+  if (POLY || d.ew_poly) {
     double ex, cx;
     const double r = r2 * rinv;
     ewald_factors(d, r2, r, ex, cx);
@@ -853,7 +854,8 @@ void launch_pair(const Launch& L, int ev, const int* cp, bool fold, bool spend) 
       else launch_pair_mixed<0, false>(L, cp, sp);
     }
   } else {
-    // the Ewald polynomials wherever every system has them
+    // with a system that has no Ewald polynomials: chosen system by system, so that
+    // the batch around a system does not change its sums
     if (L.ew_poly) {
       if (ev) launch_pair_f64<true, true>(L, cp, sp);
       else launch_pair_f64<false, true>(L, cp, sp);
