@@ -362,6 +362,15 @@ static double pair_tiles_estimate(int n, const double L[3], double rc) {
 constexpr double ENTRY_TILES = 16384.0;
 static int has_entry_list(int mixed, double tiles) { return mixed && tiles < ENTRY_TILES; }
 
+// Tiles per pair-kernel work item, from the system at its creation alone: how FP32 sums
+// are cut must depend neither on the batch around a system nor, under a barostat, on
+// the box in which its list happened to be allocated again.  A wave runs an item's tiles one after the other,
+// so a list of few items is as slow as one item: 1,000 atoms (6,000 tiles) 15.2 us
+// with 32 tiles, 9.6 with 16, 6.7 with 8.  An item costs its clusters' loads and
+// two force flushes: 227,000 atoms (2.2 M tiles) 285 us with 32, 300 with 16, 376
+// with 8; 24 systems of 1,000 to 25,000 atoms 408, 420 and 452 us a step.
+static int pair_item_tiles(double tiles) { return tiles < 16384.0 ? MIN_ITEM_TILES : tiles < 65536.0 ? 16 : 32; }
+
 int System::alloc_device() {
   const HostTopo& h = topo;
   SysDev& d = dv;
@@ -529,7 +538,9 @@ int System::alloc_device() {
   FZ_TRY(dalloc(&d.mF, (size_t)3 * n));
   FZ_TRY(dalloc(&snap, (size_t)9 * n + (F_NSLOT * sizeof(int) + 7) / 8));
   d.snap = snap;
-  d.entry_list = has_entry_list(mixed, pair_tiles_estimate(n, par.box, par.cutoff));
+  pair_tiles = pair_tiles_estimate(n, par.box, par.cutoff);
+  d.entry_list = has_entry_list(mixed, pair_tiles);
+  d.item_tiles = pair_item_tiles(pair_tiles);
   return set_column_grid(par.column_grid[0], par.column_grid[1], 1.0);
 }
 
@@ -560,14 +571,6 @@ static size_t rnd256(size_t b) { return (std::max<size_t>(1, b) + 255) & ~(size_
 // search waves per I cluster the search buffers are sized for (small systems
 // search each I cluster with several waves: more waves in flight)
 static int search_parts_of(int clusters_cap) { return clusters_cap < 8192 ? 4 : clusters_cap < 16384 ? 2 : 1; }
-
-// Tiles per pair-kernel work item, from the system alone (a system's sums must not
-// depend on the batch around it).  A wave runs an item's tiles one after the other,
-// so a list of few items is as slow as one item: 1,000 atoms (6,000 tiles) 15.2 us
-// with 32 tiles, 9.6 with 16, 6.7 with 8.  An item costs its clusters' loads and
-// two force flushes: 227,000 atoms (2.2 M tiles) 285 us with 32, 300 with 16, 376
-// with 8; 24 systems of 1,000 to 25,000 atoms 408, 420 and 452 us a step.
-static int pair_item_tiles(double tiles) { return tiles < 16384.0 ? MIN_ITEM_TILES : tiles < 65536.0 ? 16 : 32; }
 
 // Pair groups of a list of at most pairs_cap entries: an entry gives its eight j
 // slots at most, to one of three runs per pair of clusters, each with a last group
@@ -661,7 +664,6 @@ int System::alloc_neighbor_block(long long pairs_cap, int clusters_cap) {
   FZ_TRY(dalloc(&d.pg_j, ((size_t)d.n_groups_cap + 2) * 8, false));
   FZ_TRY(dalloc(&d.pg_item, items_cap((size_t)d.n_groups_cap, clusters_cap), false));
   FZ_TRY(dalloc(&d.pg_n, 1));
-  d.item_tiles = pair_item_tiles(pair_tiles_estimate(d.n_atoms, d.L, d.rc));
   return FZ_OK;
 }
 
@@ -1066,12 +1068,11 @@ int Engine::prepare() {
   for (auto* s : sys_) {
     const SysDev& d = s->dv;
     atoms_total += d.n_atoms;
-    const double t = pair_tiles_estimate(d.n_atoms, d.L, d.rc);
     if (d.entry_list) {
       L_.n_entry++;
-      chunks += 1.6 * t / PAIR_CHUNK;  // a tile of two whole clusters has fewer pairs
+      chunks += 1.6 * s->pair_tiles / PAIR_CHUNK;  // a tile of two whole clusters has fewer pairs
     } else {
-      items4 += 1.3 * t / (4.0 * pair_item_tiles(t));  // items are cut per pair of clusters: some are short
+      items4 += 1.3 * s->pair_tiles / (4.0 * d.item_tiles);  // items are cut per pair of clusters: some are short
     }
   }
   const int grid0 = items4 >= 16384.0 ? 16384 : std::max(256, ((int)items4 + 63) / 64 * 64);

@@ -66,6 +66,7 @@ struct System {
   int64_t step = 0;
   int gen = 0;  // bumped whenever device buffers are reallocated
   double self_energy = 0.0;
+  double pair_tiles = 0.0;  // estimated tiles of the pair list at creation
   double min_step = 0.0;  // adaptive minimiser step carried between calls (0 = start at the maximum)
   bool need_rebuild = true;
   // spread path that last wrote the PME accumulation grid: 0 atomic (the grid is
