@@ -572,12 +572,15 @@ static size_t rnd256(size_t b) { return (std::max<size_t>(1, b) + 255) & ~(size_
 // search each I cluster with several waves: more waves in flight)
 static int search_parts_of(int clusters_cap) { return clusters_cap < 8192 ? 4 : clusters_cap < 16384 ? 2 : 1; }
 
-// Pair groups of a list of at most pairs_cap entries: an entry gives its eight j
-// slots at most, to one of three runs per pair of clusters, each with a last group
-// of its own.  Their work items: one per MIN_ITEM_TILES tiles, two to a group, and
-// a last one per pair of clusters.
+// Room for the pair groups of a list of pairs_cap entries.  Lists have 0.40 to 0.47
+// groups per entry (waters, slabs, flat and tall boxes, cutoffs of 9 to 12); where the
+// cutoff is several times a cluster's width it can be over a half, and in the worst case
+// (no slot shared) every entry is a group: then the list grows as for want of entries.
+// A group with its items takes 52 bytes, so room for the worst case would double the
+// device memory of a large system.  Their work items: one per MIN_ITEM_TILES tiles, two
+// to a group, and a last one per pair of clusters.
 static size_t groups_cap(long long pairs_cap, int clusters_cap) {
-  return (size_t)pairs_cap + 3 * (((size_t)clusters_cap + 1) / 2);
+  return (size_t)pairs_cap / 2 + 3 * (((size_t)clusters_cap + 1) / 2);
 }
 static size_t items_cap(size_t groups, int clusters_cap) {
   return 2 * groups / MIN_ITEM_TILES + ((size_t)clusters_cap + 1) / 2;

@@ -903,6 +903,7 @@ __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S,
   if (skip_build_block(d)) return;
   __shared__ int4 keys[4][FILL_HASH / 4];
   __shared__ unsigned long long vals[4][FILL_HASH];
+  __shared__ bool fits;
   __shared__ unsigned long long need[4];  // groups (low 40 bits) and items of each wave, then their offsets
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int n = *d.n_clusters;
@@ -949,7 +950,7 @@ __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S,
   }
   if (I0 == 0 && lane == 0) {
     *d.n_pairs = total;
-    d.flags[F_NBUILD] += 1;
+    atomicAdd(d.flags + F_NBUILD, 1);
   }
   __syncthreads();
   if (merge) {
@@ -983,7 +984,11 @@ __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S,
   if (lane == 0) need[wv] = (unsigned long long)(gB + g0 + g1) | ((unsigned long long)items << 40);
   __syncthreads();
   if (threadIdx.x == 0) {
-    unsigned long long run = atomicAdd(d.pg_n, need[0] + need[1] + need[2] + need[3]);
+    const unsigned long long all = need[0] + need[1] + need[2] + need[3];
+    unsigned long long run = atomicAdd(d.pg_n, all);
+    fits = (long long)((run + all) & ((1ull << 40) - 1)) <= d.n_groups_cap;
+    // more groups than there is room for: as with more entries, no build to count
+    if (!fits && !(atomicOr(d.flags + F_OVERFLOW, OV_PAIRS) & OV_PAIRS)) atomicSub(d.flags + F_NBUILD, 1);
     for (int k = 0; k < 4; k++) {
       const unsigned long long v = need[k];
       need[k] = run;
@@ -991,6 +996,7 @@ __global__ __launch_bounds__(256) void k_pair_fill(const SysDev* __restrict__ S,
     }
   }
   __syncthreads();
+  if (!fits) return;  // the whole block
   const long long gofs = (long long)(need[wv] & ((1ull << 40) - 1));
   int4* it = d.pg_item + (need[wv] >> 40);
   // items of about equal tiles: tile t lies in group t / 2 of B or in A0, A1 after it
