@@ -92,6 +92,22 @@ def run_steps(s, n, done, reassign_every, T, seed):
     return done
 
 
+def group_tiles(s):
+    """8x8 tiles the pair kernel runs over the list held (slabs: pair groups): the
+    j slots of two neighbouring clusters' entries, those near both in groups of two
+    tiles per eight slots, those near one of them in groups of one."""
+    pairs, masks = s.cluster_pairs()
+    cl, J = pairs[:, 0].astype(np.int64), pairs[:, 1].astype(np.int64)
+    slots = masks.view(np.uint8).reshape(-1, 8) != 0
+    key, at = np.unique((cl >> 1) * (J.max() + 1) + J, return_inverse=True)
+    near = np.zeros((2, len(key), 8), bool)
+    near[cl & 1, at] = slots
+    of = key // (J.max() + 1)
+    groups = [np.ceil(np.bincount(of, n.sum(1)) / 8.0).sum()
+              for n in (near[0] & near[1], near[0] & ~near[1], near[1] & ~near[0])]
+    return int(2 * groups[0] + groups[1] + groups[2])
+
+
 def md(ctx, topo, x, p, prec, steps, warmup, seed=1):
     s = fenzi.System(ctx, topo, p, prec, xyz=x)
     T, every = p["temperature"], int(p.get("reassign_every", 0))
@@ -114,7 +130,7 @@ def md(ctx, topo, x, p, prec, steps, warmup, seed=1):
     pk = s.pair_kernel_time(20)
     out = dict(ms_per_step=ms, ns_per_day=ns_day(ms, p["dt_ps"]), temperature=e["temperature"],
                pairs_within_cutoff=int(e["pairs_within_cutoff"]), list_builds=int(e["list_builds"]), phases_ms=ph,
-               pair_tiles=int(e["pair_tiles"]),
+               list_entries=int(e["pair_tiles"]), pair_tiles=group_tiles(s),
                pair_kernel_ms=pk,
                device_bytes=s.info()["device_bytes"], autotune={k: float(v) for k, v in tuned.items()})
     return out, s
@@ -197,7 +213,7 @@ def roofline(run, prec, workload):
             "traffic": None if tr is None else tr["bytes_per_launch"],
             "traffic_source": None if tr is None else tr["source"],
             "flop_per_launch": flops, "pairs_per_launch": run["pairs_within_cutoff"],
-            "tiles_per_launch": run["pair_tiles"],
+            "tiles_per_launch": run["pair_tiles"], "list_entries": run["list_entries"],
             "in_cutoff_lane_fraction": run["pairs_within_cutoff"] / (64.0 * max(1, run["pair_tiles"])),
             "launch_ms": run["pair_kernel_ms"],
             "timing": "mean of 20 force-only launches back to back, two HIP events on the launch stream "
