@@ -1118,18 +1118,6 @@ int Engine::ensure() {
   bool stale = !prepared_ || gens_.size() != sys_.size();
   for (size_t k = 0; !stale && k < sys_.size(); k++) stale = gens_[k] != sys_[k]->gen;
   if (stale) FZ_TRY(prepare());
-  // The atomic spread adds into a zero grid, which its x pass leaves behind;
-  // the brick spread overwrites the grid and leaves its last spread there.  A
-  // member whose grid was last spread by bricks (in another engine: a batch
-  // over 64K atoms) is cleared before this engine spreads atomically.
-  for (auto* s : sys_) {
-    if (L_.pme_planes) continue;  // the plane kernels neither read nor clear the grid accumulator
-    if (!L_.spread_bricks && s->grid_mode != 0 && s->dv.Qacc) {
-      const size_t K3 = (size_t)s->dv.K[0] * s->dv.K[1] * s->dv.K[2];
-      FZ_HIP(hipMemsetAsync(s->dv.Qacc, 0, K3 * 8, L_.stream));
-    }
-    s->grid_mode = L_.spread_bricks;
-  }
   return FZ_OK;
 }
 

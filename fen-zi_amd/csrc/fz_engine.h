@@ -69,9 +69,6 @@ struct System {
   double pair_tiles = 0.0;  // estimated tiles of the pair list at creation
   double min_step = 0.0;  // adaptive minimiser step carried between calls (0 = start at the maximum)
   bool need_rebuild = true;
-  // spread path that last wrote the PME accumulation grid: 0 atomic (the grid is
-  // left zero), 1 bricks (the grid holds that spread); allocated zero
-  int grid_mode = 0;
   // Snapshot for restoring a call that failed or overflowed: 3n positions,
   // 3n velocities (as bits), 3n positions of the last list build, then the
   // status flags (F_NSLOT ints); step and minimiser step on the host.

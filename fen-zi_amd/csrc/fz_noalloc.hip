@@ -178,7 +178,7 @@ int pme_convolve_noalloc(int device, const int32_t K[3], const double box[3], do
   L.mixed = mixed;
   L.fft_nl = NL;
   L.fft_lds = fft_dyn_lds(NL, d.K, csz);
-  L.spread_bricks = 0;  // the x pass clears the accumulation grid after reading it
+  L.spread_bricks = 0;
   L.w_fftx = Work{pre + 0, (K[1] * K[2] + NL - 1) / NL};
   L.w_ffty = Work{pre + 2, K[2] * ng};
   L.w_fftz = Work{pre + 4, K[1] * ng};

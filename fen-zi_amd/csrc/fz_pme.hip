@@ -379,10 +379,10 @@ __device__ __forceinline__ const C* stage_tw(C* lds, const C* __restrict__ tw, i
 
 // x pass, forward: real grid -> half spectrum.  BRICKS: the grid's lines are summed out
 // of the bricks' blocks first (as a kernel of its own, through the grid: 39 + 15 us at
-// 144^3; this 46, without the launch between); otherwise the grid is cleared after reading when asked.
+// 144^3; this 46, without the launch between); otherwise the grid is read and cleared,
+// as the next atomic spread needs it.
 template <bool MIXED, bool BRICKS>
-__global__ __launch_bounds__(256) void k_fft_x_r2c(const SysDev* __restrict__ S, int nsys, const int* __restrict__ pre, int NL,
-                                                    int clear) {
+__global__ __launch_bounds__(256) void k_fft_x_r2c(const SysDev* __restrict__ S, int nsys, const int* __restrict__ pre, int NL) {
   using R = typename std::conditional<MIXED, float, double>::type;
   using C = typename C2<R>::t;
   using A = typename std::conditional<MIXED, unsigned long long, double>::type;
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void k_fft_x_r2c(const SysDev* __restrict__ S,
         const size_t g = (size_t)(l0 + line) * K0 + x;
         A* Q = (A*)d.Qacc;
         v.x = MIXED ? (R)from_fixed_acc((unsigned long long)Q[g]) : (R)Q[g];
-        if (clear) Q[g] = A(0);
+        Q[g] = A(0);
         return v;
       },
       [&](int line, int kx, C v, C*) {
@@ -864,10 +864,8 @@ template <bool MIXED>
 static void launch_fft_passes(const Launch& L, bool ev, int mode, bool bricks) {
   const size_t lds = L.fft_lds;
   const int NL = L.fft_nl;
-  // the atomic spread adds into a zero grid: the x pass clears it after reading
-  if (bricks) hipLaunchKernelGGL((k_fft_x_r2c<MIXED, true>), dim3(L.w_fftx.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_fftx.pre, NL, 0);
-  else hipLaunchKernelGGL((k_fft_x_r2c<MIXED, false>), dim3(L.w_fftx.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_fftx.pre, NL,
-                          L.spread_bricks ? 0 : 1);
+  if (bricks) hipLaunchKernelGGL((k_fft_x_r2c<MIXED, true>), dim3(L.w_fftx.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_fftx.pre, NL);
+  else hipLaunchKernelGGL((k_fft_x_r2c<MIXED, false>), dim3(L.w_fftx.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_fftx.pre, NL);
   hipLaunchKernelGGL(k_fft_y<MIXED>, dim3(L.w_ffty.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_ffty.pre, NL, -1);
   if (ev) hipLaunchKernelGGL((k_fft_z_conv<MIXED, true>), dim3(L.w_fftz.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_fftz.pre, NL, mode);
   else hipLaunchKernelGGL((k_fft_z_conv<MIXED, false>), dim3(L.w_fftz.total), dim3(256), lds, L.stream, L.d_sys, L.nsys, L.w_fftz.pre, NL, mode);

@@ -187,7 +187,7 @@ struct SysDev {
   float2 *lj_ah;                          // [n_types]
   double2 *lj14;                          // 1-4 (eps, sigma^2)
   // ---- PME --------------------------------------------------------------------
-  void *Qacc;      // K0*K1*K2 accumulators (double or fixed int64)
+  void *Qacc;      // K0*K1*K2 accumulators (double or fixed int64) of the atomic spread; zero between evaluations
   void *Qc;        // complex half grid [K2][K1][Kxh] (float2 / double2)
   void *phi;       // real potential grid [K2][K1][K0] (float / double)
   double *pme_bsp; // per-axis |b(m)|^2, [K0 + K1 + K2]
@@ -198,7 +198,7 @@ struct SysDev {
   // Charge spreading by grid bricks of 8^3 points: atoms are counted and
   // ordered by the brick holding the first point of their 4^3 stencil, each
   // brick's stencils are summed in LDS over its (8+3)^3 block, and the blocks
-  // overlapping a grid point are added into Qacc.
+  // overlapping a grid point are added by the first transform's lines.
   int nbr[3];      // bricks per axis, ceil(K_d / 8)
   int n_bricks;
   int *br_cnt;     // [n_bricks] atoms per brick (counted each step, cleared by the scan)
