@@ -13,13 +13,13 @@ const char* last_error();
 }
 
 struct fz_system {
-  fz_ctx* ctx;
+  int device;  // the context's (it may be destroyed before its systems: a collected cycle ends in any order)
   System sys;
   std::unique_ptr<Engine> eng;
 };
 
 struct fz_batch {
-  fz_ctx* ctx;
+  int device;
   std::vector<fz_system*> members;
   std::unique_ptr<Engine> eng;
 };
@@ -56,7 +56,7 @@ int fz_system_create(fz_ctx* ctx, const fz_topology* topo, const fz_params* par,
   if (!ctx || !topo || !par || !out) return set_error(FZ_ERR_ARG, "null argument");
   FZ_HIP(hipSetDevice(ctx->device));
   auto* s = new fz_system();
-  s->ctx = ctx;
+  s->device = ctx->device;
   int r = s->sys.init(topo, par, precision, ctx->device);
   if (r != FZ_OK) { delete s; return r; }
   s->eng.reset(new Engine(ctx->device, {&s->sys}));
@@ -69,7 +69,7 @@ int fz_system_create(fz_ctx* ctx, const fz_topology* topo, const fz_params* par,
 
 void fz_system_destroy(fz_system* s) {
   if (!s) return;
-  (void)hipSetDevice(s->ctx->device);
+  (void)hipSetDevice(s->device);
   s->eng.reset();
   delete s;
 }
@@ -77,7 +77,7 @@ void fz_system_destroy(fz_system* s) {
 int fz_set_state(fz_system* s, const double* xyz, const double* vel) {
   FZ_GUARD_BEGIN
   if (!s || !xyz) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->sys.upload_positions(xyz));
   FZ_TRY(s->sys.upload_velocities(vel));
   FZ_TRY(s->eng->forces(true));
@@ -88,7 +88,7 @@ int fz_set_state(fz_system* s, const double* xyz, const double* vel) {
 int fz_get_state(fz_system* s, double* xyz, double* vel) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->eng->sync());
   return s->sys.download_state(xyz, vel, nullptr);
   FZ_GUARD_END
@@ -97,7 +97,7 @@ int fz_get_state(fz_system* s, double* xyz, double* vel) {
 int fz_set_fixed_positions(fz_system* s, const uint64_t* u) {
   FZ_GUARD_BEGIN
   if (!s || !u) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->sys.upload_fixed(u));
   FZ_TRY(s->eng->forces(true));
   return s->eng->npt_reset_virial();
@@ -107,7 +107,7 @@ int fz_set_fixed_positions(fz_system* s, const uint64_t* u) {
 int fz_set_barostat(fz_system* s, double pref_atm, double piston_mass) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->eng->sync());
   FZ_TRY(s->sys.set_barostat(pref_atm, piston_mass));
   FZ_TRY(s->eng->forces(true));
@@ -133,7 +133,7 @@ int fz_get_barostat(fz_system* s, double* box, double* state) {
 int fz_get_fixed_positions(fz_system* s, uint64_t* u) {
   FZ_GUARD_BEGIN
   if (!s || !u) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->eng->sync());
   return s->sys.download_state(nullptr, nullptr, u);
   FZ_GUARD_END
@@ -142,7 +142,7 @@ int fz_get_fixed_positions(fz_system* s, uint64_t* u) {
 int fz_reassign_velocities(fz_system* s, double T, uint64_t seed, uint64_t counter) {
   FZ_GUARD_BEGIN
   if (!s || !(T >= 0)) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->maxwell(T, seed, counter);
   FZ_GUARD_END
 }
@@ -150,7 +150,7 @@ int fz_reassign_velocities(fz_system* s, double T, uint64_t seed, uint64_t count
 int fz_set_fixed_atoms(fz_system* s, const uint8_t* fixed) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->sys.set_fixed(fixed);
   FZ_GUARD_END
 }
@@ -158,7 +158,7 @@ int fz_set_fixed_atoms(fz_system* s, const uint8_t* fixed) {
 int fz_set_com_restraint(fz_system* s, const int32_t* group, const double dist[3], double fc) {
   FZ_GUARD_BEGIN
   if (!s || (group && !dist)) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->sys.set_com_restraint(group, dist, fc);
   FZ_GUARD_END
 }
@@ -166,7 +166,7 @@ int fz_set_com_restraint(fz_system* s, const int32_t* group, const double dist[3
 int fz_compute_forces(fz_system* s, double* f, fz_energies* e) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->eng->forces(true));
   if (f) FZ_TRY(s->sys.download_forces(f));
   if (e) FZ_TRY(s->sys.energies(e));
@@ -177,7 +177,7 @@ int fz_compute_forces(fz_system* s, double* f, fz_energies* e) {
 int fz_step(fz_system* s, int nsteps) {
   FZ_GUARD_BEGIN
   if (!s || nsteps < 0) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->steps(nsteps);
   FZ_GUARD_END
 }
@@ -185,7 +185,7 @@ int fz_step(fz_system* s, int nsteps) {
 int fz_set_neighbor_capacity(fz_system* s, int64_t pairs_cap, int32_t clusters_cap) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->set_capacity(0, pairs_cap, clusters_cap);
   FZ_GUARD_END
 }
@@ -193,7 +193,7 @@ int fz_set_neighbor_capacity(fz_system* s, int64_t pairs_cap, int32_t clusters_c
 int fz_phase_times(fz_system* s, int nsteps, double* ms) {
   FZ_GUARD_BEGIN
   if (!s || nsteps <= 0 || !ms) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->phase_times(nsteps, ms);
   FZ_GUARD_END
 }
@@ -201,7 +201,7 @@ int fz_phase_times(fz_system* s, int nsteps, double* ms) {
 int fz_pair_kernel_time(fz_system* s, int reps, double* ms) {
   FZ_GUARD_BEGIN
   if (!s || reps <= 0 || !ms) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->pair_kernel_time(reps, ms);
   FZ_GUARD_END
 }
@@ -209,7 +209,7 @@ int fz_pair_kernel_time(fz_system* s, int reps, double* ms) {
 int fz_autotune(fz_system* s, int nsteps, double* out) {
   FZ_GUARD_BEGIN
   if (!s || nsteps <= 0 || !out) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->autotune(nsteps, out);
   FZ_GUARD_END
 }
@@ -217,7 +217,7 @@ int fz_autotune(fz_system* s, int nsteps, double* out) {
 int fz_set_launch(fz_system* s, int nl, int grid, int pme_path, int32_t* out) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->set_launch(nl, grid, pme_path, out);
   FZ_GUARD_END
 }
@@ -225,7 +225,7 @@ int fz_set_launch(fz_system* s, int nl, int grid, int pme_path, int32_t* out) {
 int fz_batch_set_launch(fz_batch* b, int nl, int grid, int pme_path, int32_t* out) {
   FZ_GUARD_BEGIN
   if (!b) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(b->ctx->device));
+  FZ_HIP(hipSetDevice(b->device));
   return b->eng->set_launch(nl, grid, pme_path, out);
   FZ_GUARD_END
 }
@@ -233,7 +233,7 @@ int fz_batch_set_launch(fz_batch* b, int nl, int grid, int pme_path, int32_t* ou
 int fz_batch_phase_times(fz_batch* b, int nsteps, double* ms) {
   FZ_GUARD_BEGIN
   if (!b || nsteps <= 0 || !ms) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(b->ctx->device));
+  FZ_HIP(hipSetDevice(b->device));
   return b->eng->phase_times(nsteps, ms);
   FZ_GUARD_END
 }
@@ -241,7 +241,7 @@ int fz_batch_phase_times(fz_batch* b, int nsteps, double* ms) {
 int fz_batch_autotune(fz_batch* b, int nsteps, double* out) {
   FZ_GUARD_BEGIN
   if (!b || nsteps <= 0 || !out) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(b->ctx->device));
+  FZ_HIP(hipSetDevice(b->device));
   return b->eng->autotune(nsteps, out);
   FZ_GUARD_END
 }
@@ -263,7 +263,7 @@ int fz_get_cluster_layout(fz_system* s, int32_t* ncx_ncy, int32_t* atom_column, 
                           int64_t slot_cap, int64_t* n_slots) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->eng->sync());
   const SysDev& d = s->sys.dv;
   int ncl = 0;
@@ -282,7 +282,7 @@ int fz_get_cluster_layout(fz_system* s, int32_t* ncx_ncy, int32_t* atom_column, 
 int64_t fz_get_cluster_pairs(fz_system* s, int32_t* pairs, uint64_t* masks, int64_t cap) {
   FZ_GUARD_BEGIN
   if (!s) return set_error(FZ_ERR_ARG, "null argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   FZ_TRY(s->eng->sync());
   const SysDev& d = s->sys.dv;
   long long np = 0;
@@ -318,10 +318,10 @@ int fz_batch_create(fz_ctx* ctx, fz_system* const* systems, int n, fz_batch** ou
   if (!ctx || !systems || n <= 0 || !out) return set_error(FZ_ERR_ARG, "invalid argument");
   FZ_HIP(hipSetDevice(ctx->device));
   auto* b = new fz_batch();
-  b->ctx = ctx;
+  b->device = ctx->device;
   std::vector<System*> ss;
   for (int i = 0; i < n; i++) {
-    if (!systems[i] || systems[i]->ctx->device != ctx->device) { delete b; return set_error(FZ_ERR_ARG, "system %d invalid", i); }
+    if (!systems[i] || systems[i]->device != ctx->device) { delete b; return set_error(FZ_ERR_ARG, "system %d invalid", i); }
     b->members.push_back(systems[i]);
     ss.push_back(&systems[i]->sys);
   }
@@ -336,14 +336,14 @@ int fz_batch_create(fz_ctx* ctx, fz_system* const* systems, int n, fz_batch** ou
 int fz_batch_step(fz_batch* b, int nsteps) {
   FZ_GUARD_BEGIN
   if (!b || nsteps < 0) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(b->ctx->device));
+  FZ_HIP(hipSetDevice(b->device));
   return b->eng->steps(nsteps);
   FZ_GUARD_END
 }
 
 void fz_batch_destroy(fz_batch* b) {
   if (!b) return;
-  (void)hipSetDevice(b->ctx->device);
+  (void)hipSetDevice(b->device);
   b->eng.reset();
   delete b;
 }
@@ -351,7 +351,7 @@ void fz_batch_destroy(fz_batch* b) {
 int fz_minimize(fz_system* s, int nsteps, double max_step) {
   FZ_GUARD_BEGIN
   if (!s || nsteps < 0 || !(max_step > 0)) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->minimize(nsteps, max_step);
   FZ_GUARD_END
 }
@@ -359,7 +359,7 @@ int fz_minimize(fz_system* s, int nsteps, double max_step) {
 int fz_batch_minimize(fz_batch* b, int nsteps, double max_step) {
   FZ_GUARD_BEGIN
   if (!b || nsteps < 0 || !(max_step > 0)) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(b->ctx->device));
+  FZ_HIP(hipSetDevice(b->device));
   return b->eng->minimize(nsteps, max_step);
   FZ_GUARD_END
 }
@@ -373,7 +373,7 @@ static bool min_params_ok(const fz_min_params* p) {
 int fz_minimize_ex(fz_system* s, int nsteps, const fz_min_params* p) {
   FZ_GUARD_BEGIN
   if (!s || nsteps < 0 || !min_params_ok(p)) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(s->ctx->device));
+  FZ_HIP(hipSetDevice(s->device));
   return s->eng->minimize_ref(nsteps, *p);
   FZ_GUARD_END
 }
@@ -381,7 +381,7 @@ int fz_minimize_ex(fz_system* s, int nsteps, const fz_min_params* p) {
 int fz_batch_minimize_ex(fz_batch* b, int nsteps, const fz_min_params* p) {
   FZ_GUARD_BEGIN
   if (!b || nsteps < 0 || !min_params_ok(p)) return set_error(FZ_ERR_ARG, "invalid argument");
-  FZ_HIP(hipSetDevice(b->ctx->device));
+  FZ_HIP(hipSetDevice(b->device));
   return b->eng->minimize_ref(nsteps, *p);
   FZ_GUARD_END
 }
