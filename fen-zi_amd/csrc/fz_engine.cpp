@@ -1814,7 +1814,7 @@ int Engine::autotune(int nsteps, double* out) {
   bool explicit_grid = true;
   for (auto* s : sys_) explicit_grid = explicit_grid && s->par.column_grid[0] > 0 && s->par.column_grid[1] > 0;
   double best_f = 1.0, best_ms = 1e30, ms = 0;
-  int best_nl = 16, best_grid = 2048;
+  int best_nl = 16, best_grid = 0;  // 0: the default grid, for the size of the lists
   int rc = FZ_OK;
   std::vector<double> widths = {0.8, 0.9, 1.0, 1.15, 1.3};
   if (explicit_grid) widths = {1.0};
@@ -1840,7 +1840,7 @@ int Engine::autotune(int nsteps, double* out) {
   }
   FZ_TRY(configure(best_f, best_nl, best_grid));
   FZ_TRY(forces(true));
-  out[0] = best_f; out[1] = best_nl; out[2] = best_grid; out[3] = best_ms;
+  out[0] = best_f; out[1] = best_nl; out[2] = L_.pair_grid; out[3] = best_ms;
   return FZ_OK;
 }
 
