@@ -108,7 +108,7 @@ def group_tiles(s):
     return int(2 * groups[0] + groups[1] + groups[2])
 
 
-def md(ctx, topo, x, p, prec, steps, warmup, seed=1):
+def md(ctx, topo, x, p, prec, steps, warmup, seed=1, tune=True):
     s = fenzi.System(ctx, topo, p, prec, xyz=x)
     T, every = p["temperature"], int(p.get("reassign_every", 0))
     s.reassign_velocities(T, seed, 0)
@@ -116,7 +116,7 @@ def md(ctx, topo, x, p, prec, steps, warmup, seed=1):
     # the library's autotuner; it times trial steps and restores the state.  It
     # runs before the warm-up, so that the warm-up captures the step graphs of
     # the chosen shapes and the timed steps replay them.
-    tuned = s.autotune(40)
+    tuned = s.autotune(40) if tune else {}
     done = run_steps(s, max(2, warmup), 0, every, T, seed)
     # fz_step returns once the device has finished (it reads the status flags)
     t0 = time.perf_counter()
@@ -366,12 +366,13 @@ def serving(ctx, jobs, arrival, md_steps, budget, chunk):
 
 def profile_run(a):
     """Mixed leg of one slab (--profile-workload 1: 17K, 2: 230K; graph-replayed
-    steps, then the eager phase timing) followed by one device-to-device copy of
+    steps in the default launch shapes, since trial steps timed under a profiler
+    choose others, then the eager phase timing) followed by one device-to-device copy of
     a known size, so that the same counter run gives the counter's reading for a
     plain copy."""
     ctx = fenzi.Context(0)
     topo1, x1, p1 = prepare(ctx, a.profile_workload, a.min_steps)
-    r1m, s = md(ctx, topo1, x1, p1, fenzi.MIXED, a.steps, a.warmup)
+    r1m, s = md(ctx, topo1, x1, p1, fenzi.MIXED, a.steps, a.warmup, tune=False)
     s.close()
     log("%d atoms mixed: %.3f ms/step; pair %.4f ms per launch (%.4f ms with the phase events), %d pairs" % (
         topo1["n_atoms"], r1m["ms_per_step"], r1m["pair_kernel_ms"], r1m["phases_ms"]["pair"], r1m["pairs_within_cutoff"]))
