@@ -59,12 +59,15 @@ __device__ __forceinline__ bool skip_build_block(const SysDev& d) {
 
 // Last block done: each of the system's nblocks blocks takes a ticket once its
 // device-scope atomics are performed; the block that draws the last ticket sees every
-// other block's atomics (read with agent_load, past its own caches) and runs the
-// system's single-block step (no block ever waits for another).  The counter is left
-// at zero for the next launch.  Plain stores are not ordered by this: a release fence
-// would be, but writes back the XCD's whole L2, of the order of 0.5 us per block and
-// XCD (50,000 atoms: 25 us for the count with it, 6 without).
-__device__ __forceinline__ bool last_block(unsigned* ctr, int nblocks) {
+// other block's atomics, if it reads them with agent_load (past its own caches), and
+// runs the system's single-block step (no block ever waits for another).  The counter
+// is left at zero for the next launch.
+// Only atomics: a wave's s_waitcnt waits until its atomics have been performed where
+// agent_load reads, which holds for this target and not for the language's memory
+// model; plain stores stay in the XCD's L2.  A step that reads plain stores needs a
+// release fence before the ticket, which writes that L2 back, of the order of 0.5 us per
+// block and XCD (50,000 atoms: 25 us for the count with it, 6 without).
+__device__ __forceinline__ bool last_block_of_atomics(unsigned* ctr, int nblocks) {
   __shared__ int last;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(256) void k_bin_count(const SysDev* __restrict__ S,
       if (v) atomicAdd(d.col_count + CNT_LINE * k, v);
     }
   }
-  if (FUSED && last_block(d.tick + 0, pre[s_ + 1] - pre[s_])) col_scan_block(d);
+  if (FUSED && last_block_of_atomics(d.tick + 0, pre[s_ + 1] - pre[s_])) col_scan_block(d);
 }
 
 // one block per system

@@ -9,8 +9,9 @@
 // pair group: lane l holds i = l & 7, j = l >> 3.  j forces are summed over the 8
 // lanes that share j (xor 1, 2, 4), tile by tile, and added once per group (in the
 // mixed form the tiles' sums are added in fixed point: a sum of both in FP32 would
-// round once more and saved nothing, 227,000 atoms 288 and 290 us); i forces stay in registers for the whole work item (a run of the groups
-// of two clusters), then are reduced over lanes l, l+8, ... (xor 8, 16, 32).
+// round once more and saved nothing, 227,000 atoms 288 and 290 us); i forces stay in
+// registers for the whole work item (a run of the groups of two clusters), then are
+// reduced over lanes l, l+8, ... (xor 8, 16, 32).
 //
 // What bounds it: vector issue (every lane of a tile costs the same whether its
 // pair is inside the cutoff or not), and the j-force atomics, which resolve beyond
@@ -18,11 +19,12 @@
 // A tile of two whole clusters carries a pair inside the cutoff in 0.33 of its
 // lanes (cutoff 12, list 13.5; 0.29 at 10 / 11.5): most j clusters of an entry
 // reach the list distance with some of their atoms only.  The groups hold the j
-// slots one by one, without those no atom of the i cluster is near: 0.48 and 0.42
-// of the lanes, a third fewer tiles.  With a list per i cluster the atomics then
+// slots one by one, without those no atom of the i cluster is near: 0.46 and 0.41
+// of the lanes, three tenths fewer tiles.  With a list per i cluster the atomics then
 // bound the kernel (227,000 atoms: 400 us, 234 without them); two neighbouring
-// clusters share their groups, which leaves 0.64 of the cache lines.  A j slot's record is one 32-byte sector, gathered with a
-// per-lane byte offset that the list holds ready (no address arithmetic).
+// clusters share their groups, which leaves 0.64 of the cache lines.  A j slot's
+// record is one 32-byte sector, gathered with a per-lane byte offset that the list
+// holds ready (no address arithmetic).
 //
 // Mixed form: int32 fixed-point displacements (the top 32 bits of the 64-bit
 // fractions; int32 wrap-around is the minimum image), FP32 arithmetic, own
@@ -590,8 +592,9 @@ __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S
 // entries each, all their records loaded before the first is used, and leave the i
 // terms in LDS; then one wave per component adds them up entry by entry.
 //
-// What bounds it: latency (1,000 atoms: 280 chunks).  A wave per chunk, as one would
-// run them with more of them than the chip has waves, took 15.2 us at 1,000 atoms.
+// What bounds it: latency (1,000 atoms: 274 chunks).  12.2 us at 1,000 atoms, back to
+// back; a wave per chunk took 15.2, pair groups 6.7, and eight or sixteen waves 10.7 and
+// 10.5.  A step (the PME kernels beside it take longer) is the same with all but the first.
 constexpr int ENTRY_WAVE = PAIR_CHUNK / 4;  // entries of a wave
 
 template <int EV, bool SEP>
