@@ -369,6 +369,11 @@ static double pair_tiles_estimate(int n, const double L[3], double rc) {
 // the pair kernel's arithmetic and atomics, of which the groups need a third less.
 constexpr double ENTRY_TILES = 16384.0;
 static int has_entry_list(int mixed, double tiles) { return mixed && tiles < ENTRY_TILES; }
+// Launches of this many chunks of such lists or more run a wave per chunk, others a
+// workgroup.  A step of 2, 8, 12, 24 and 64 systems of 1,000 and 2,000 atoms (400 chunks
+// each on average): workgroups 71, 102, 118, 164 and 347 us, waves 80, 103, 116, 155 and
+// 262 (pair groups 71, 100, 114, 145 and 263).
+constexpr double ENTRY_WAVE_CHUNKS = 4096.0;
 
 // Tiles per pair-kernel work item, from the system at its creation alone: how FP32 sums
 // are cut must depend neither on the batch around a system nor, under a barostat, on
@@ -1088,7 +1093,9 @@ int Engine::prepare() {
   }
   const int grid0 = items4 >= 16384.0 ? 16384 : std::max(256, ((int)items4 + 63) / 64 * 64);
   L_.pair_grid = tuned_grid_ > 0 ? tuned_grid_ : grid0;
-  L_.entry_grid = tuned_grid_ > 0 ? tuned_grid_ : chunks >= 8192.0 ? 8192 : std::max(64, (int)chunks);
+  L_.entry_waves = chunks >= ENTRY_WAVE_CHUNKS;
+  const double blocks = L_.entry_waves ? chunks / 4.0 : chunks;
+  L_.entry_grid = tuned_grid_ > 0 ? tuned_grid_ : blocks >= 8192.0 ? 8192 : std::max(64, (int)blocks);
   // Spread by bricks from 24K atoms per launch; below, the single atomic kernel is
   // cheaper than the brick pipeline's four launches.  Same grid either way.  Steps,
   // atomics -> bricks: 17,000 atoms 102 -> 105 us, 21,000 113 -> 114, 42,000 161 -> 138,

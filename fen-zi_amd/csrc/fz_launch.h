@@ -80,6 +80,7 @@ struct Launch {
   int pair_grid = 0;         // persistent pair-kernel blocks
   int n_entry = 0;           // systems with an entry list (a kernel of their own)
   int entry_grid = 0;        // its blocks
+  int entry_waves = 0;       // a wave per chunk (1) or a workgroup (0)
   int fft_lds = 0;           // dynamic LDS bytes for the FFT kernels
   int fft_nl = 16;           // lines per FFT workgroup
   int lj_sep = 0;            // every system follows the LJ combination rule

@@ -310,6 +310,11 @@ __device__ __forceinline__ int work_items(const SysDev* __restrict__ S, int nsys
   return S[0].flags[F_OVERFLOW] ? 0 : (int)(*S[0].pg_n >> 40);
 }
 
+__device__ __forceinline__ int entry_items(const SysDev* __restrict__ S, int nsys, const int* __restrict__ entry_pre) {
+  if (nsys > 1) return entry_pre[nsys];
+  return S[0].flags[F_OVERFLOW] ? 0 : entry_chunks(S[0]);
+}
+
 // One i cluster of a work item in registers (mixed form).
 struct ICluster {
   int x, y, z, t;      // position top words, LJ table row
@@ -592,9 +597,10 @@ __global__ __launch_bounds__(256) void k_pair_mixed(const SysDev* __restrict__ S
 // entries each, all their records loaded before the first is used, and leave the i
 // terms in LDS; then one wave per component adds them up entry by entry.
 //
-// What bounds it: latency (1,000 atoms: 274 chunks).  12.2 us at 1,000 atoms, back to
-// back; a wave per chunk took 15.2, pair groups 6.7, and eight or sixteen waves 10.7 and
-// 10.5.  A step (the PME kernels beside it take longer) is the same with all but the first.
+// What bounds it: latency (1,000 atoms: 274 chunks).  8 to 12 us at 1,000 atoms, back to
+// back; a wave per chunk takes 18 (the step 66 us, 54 with this), pair groups 6.7, and
+// eight or sixteen waves save 1.5 us, which no step shows (the PME kernels beside it take
+// longer).
 constexpr int ENTRY_WAVE = PAIR_CHUNK / 4;  // entries of a wave
 
 template <int EV, bool SEP>
@@ -604,7 +610,7 @@ __global__ __launch_bounds__(256) void k_pair_entry(const SysDev* __restrict__ S
   __shared__ float term[PAIR_CHUNK][3][64];
   const int lane = threadIdx.x & 63, il = lane & 7, jl = lane >> 3, wv = rfl(threadIdx.x >> 6);
   chunk_pre += nsys + 1;  // the entry lists' prefix
-  const int total = rfl(nsys > 1 ? chunk_pre[nsys] : S[0].flags[F_OVERFLOW] ? 0 : entry_chunks(S[0]));
+  const int total = rfl(entry_items(S, nsys, chunk_pre));
   int evs = -1;
   EvAcc ev;
   ev.zero();
@@ -688,6 +694,94 @@ __global__ __launch_bounds__(256) void k_pair_entry(const SysDev* __restrict__ S
       flush();
     }
     __syncthreads();
+    if (EV) ev.add_item(cev, lane);
+  }
+  if (EV && evs >= 0) ev.flush(S[evs], lane);
+}
+
+// The same sums with a wave per chunk, for launches of many chunks (ENTRY_WAVE_CHUNKS):
+// no terms pass through LDS and no wave waits for another.
+template <int EV, bool SEP>
+__global__ __launch_bounds__(256) void k_pair_entry_wave(const SysDev* __restrict__ S, int nsys, const int* __restrict__ chunk_pre,
+                                                         int spend) {
+  if (spend && blockIdx.x == 0 && threadIdx.x == 0) S[0].flags[F_REBUILD] = 0;
+  const int lane = threadIdx.x & 63, il = lane & 7, jl = lane >> 3;
+  chunk_pre += nsys + 1;  // the entry lists' prefix
+  const int total = rfl(entry_items(S, nsys, chunk_pre));
+  const int nw = gridDim.x * 4;
+  int evs = -1;
+  EvAcc ev;
+  ev.zero();
+  for (int w = rfl(blockIdx.x * 4 + (threadIdx.x >> 6)); w < total; w += nw) {
+    const int s = nsys == 1 ? 0 : rfl(locate(chunk_pre, nsys, w));
+    const int wk = nsys == 1 ? w : w - chunk_pre[s];
+    const SysDev& d = S[s];
+    if (EV && s != evs) {
+      if (evs >= 0) ev.flush(S[evs], lane);
+      ev.zero();
+      evs = s;
+    }
+    double cev[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    const long long np = *d.n_pairs, e0 = (long long)wk * PAIR_CHUNK;
+    const int ne = rfl((int)(np - e0 < PAIR_CHUNK ? np - e0 : PAIR_CHUNK));
+    if (EV && wk == 0) ev.ntl += np;
+    const __amdgpu_buffer_rsrc_t xsr = raw_rsrc(d.xs, (unsigned)d.n_slots_cap * SLOT_BYTES);
+    const CI2* ent = (const CI2*)(d.pl_ij + e0);
+    const CU64* msk = (const CU64*)(d.pl_mask + e0);
+    const GF2* lj = (const GF2*)d.lj32;
+    FZ_GLOBAL char* Fb = (FZ_GLOBAL char*)d.Fs;
+    const PairConst pc(d);
+    const unsigned ioff = (unsigned)il * SLOT_BYTES, joff = (unsigned)jl * SLOT_BYTES;
+    const unsigned foff = joff + (unsigned)(lane & 7) * 8u;
+    ICluster ic;
+    float fi[3];
+    int I = -1;
+    v2i en = ent[0];
+    unsigned Js = (unsigned)en.y * (CLUSTER * SLOT_BYTES);
+    v4i xjn = buf_ld4(xsr, joff, Js);
+    v2f pjn = buf_ld2(xsr, joff + 16u, Js);
+    // j cluster one entry ahead, the j-force atomic one late (as in k_pair_mixed)
+    unsigned long long pend_m = 0ull, pend_v = 0ull;
+    unsigned pend_o = 0u;
+    for (int k = 0; k < ne; k++) {
+      const int Ik = rfl(en.x);
+      const unsigned long long m = msk[k];
+      const unsigned Jk = Js;
+      const v4i xj = xjn;
+      const v2f pj = pjn;
+      en = ent[min(k + 1, ne - 1)];
+      Js = (unsigned)en.y * (CLUSTER * SLOT_BYTES);
+      xjn = buf_ld4(xsr, joff, Js);
+      pjn = buf_ld2(xsr, joff + 16u, Js);
+      if (__builtin_amdgcn_inverse_ballot_w64(pend_m)) atomic_add_g((GU64*)(Fb + pend_o), pend_v);
+      if (Ik != I) {
+        const unsigned Is = (unsigned)Ik * (CLUSTER * SLOT_BYTES);
+        const v4i v = buf_ld4(xsr, ioff, Is);
+        const v2f lp = buf_ld2(xsr, ioff + 16u, Is);
+        if (I >= 0) flush_i(Fb, I, lane, fi[0], fi[1], fi[2]);
+        I = Ik;
+        ic.set(v, lp, d.n_types);
+        // the i loads consumed here: one in flight where this branch rejoins the loop
+        // would make every tile wait for all memory operations
+        __asm__ volatile("" ::"v"(ic.q), "v"(ic.x), "v"(ic.y), "v"(ic.z), "v"(ic.p.x), "v"(ic.p.y));
+        fi[0] = fi[1] = fi[2] = 0.f;
+      }
+      float fx, fy, fz;
+      const unsigned long long actm = tile_mixed<EV, SEP>(d, pc, lj, m, ic, xj, pj, fx, fy, fz, cev, ev.npr);
+      sub3_rn(fi, fx, fy, fz);
+      red8x3(fx, fy, fz);
+      const int c = lane & 7;
+      pend_v = fixed_f32(c == 0 ? fx : (c == 1 ? fy : fz));
+      pend_m = byte_any3(actm);
+      pend_o = Jk + foff;
+      if (EV && (k + 1) % ENTRY_WAVE == 0) {  // energies by the same eight entries as a workgroup's waves
+        ev.add_item(cev, lane);
+#pragma unroll
+        for (int q = 0; q < 8; q++) cev[q] = 0.0;
+      }
+    }
+    if (__builtin_amdgcn_inverse_ballot_w64(pend_m)) atomic_add_g((GU64*)(Fb + pend_o), pend_v);
+    flush_i(Fb, I, lane, fi[0], fi[1], fi[2]);
     if (EV) ev.add_item(cev, lane);
   }
   if (EV && evs >= 0) ev.flush(S[evs], lane);
@@ -831,7 +925,9 @@ template <int EV, bool SEP>
 static void launch_pair_mixed(const Launch& L, const int* cp, int sp) {
   if (L.n_entry < L.nsys)
     hipLaunchKernelGGL((k_pair_mixed<EV, SEP>), dim3(L.pair_grid), dim3(256), 0, L.stream, L.d_sys, L.nsys, cp, sp);
-  if (L.n_entry > 0)
+  if (L.n_entry > 0 && L.entry_waves)
+    hipLaunchKernelGGL((k_pair_entry_wave<EV, SEP>), dim3(L.entry_grid), dim3(256), 0, L.stream, L.d_sys, L.nsys, cp, sp);
+  else if (L.n_entry > 0)
     hipLaunchKernelGGL((k_pair_entry<EV, SEP>), dim3(L.entry_grid), dim3(256), 0, L.stream, L.d_sys, L.nsys, cp, sp);
 }
 

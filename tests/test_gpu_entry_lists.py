@@ -81,3 +81,30 @@ def test_batch_of_both_kinds_matches_its_members_alone(ctx):
             assert np.array_equal(a.get_state()[1], m.get_state()[1])
             assert a.energies()["potential"] == m.energies()["potential"]
     b.close()
+
+
+def test_batch_with_a_wave_per_chunk_matches_its_members_alone(ctx):
+    """Many chunks in one launch (about 800 estimated per member, from 4,096 on a wave
+    each), an odd and a tiny list among them."""
+    alone, members = [], []
+    for k, n in enumerate(["below"] * 6 + ["a_chunk", "one_entry"]):
+        topo, xyz, params = _water(*SIZES[n])
+        for group in (alone, members):
+            s = fenzi.System(ctx, topo, params, fenzi.MIXED, xyz=xyz)
+            s.reassign_velocities(300.0, 40 + k, 0)
+            group.append(s)
+    b = fenzi.Batch(ctx, members)
+    b.step(30)
+    for a, m in zip(alone, members):
+        a.step(30)
+        assert np.array_equal(a.get_fixed(), m.get_fixed())
+        assert np.array_equal(a.get_state()[1], m.get_state()[1])
+        ea, em = a.energies(), m.energies()
+        for k in ("potential", "vdw", "elec", "pairs_within_cutoff", "pair_tiles", "list_builds"):
+            assert ea[k] == em[k], k
+    b.minimize(2, 0.02)  # the other energy levels
+    for a, m in zip(alone, members):
+        a.minimize(2, 0.02)
+        assert np.array_equal(a.get_fixed(), m.get_fixed())
+        assert a.energies()["potential"] == m.energies()["potential"]
+    b.close()
