@@ -364,9 +364,11 @@ static double pair_tiles_estimate(int n, const double L[3], double rc) {
   return 0.5 * n * (4.0 / 3.0 * kPi * rc * rc * rc * rho) / 30.0;
 }
 
-// Systems of up to this many tiles keep an entry list in the mixed form (reason at
-// k_pair_entry): up to about 2,700 atoms at a cutoff of 10.  Larger ones are bound by
-// the pair kernel's arithmetic and atomics, of which the groups need a third less.
+// Systems of fewer than this many tiles keep an entry list in the mixed form (reason at
+// k_pair_entry): up to about 2,700 atoms at a cutoff of 10, where it costs a step 1 %.
+// Larger ones wait for the pair kernel, which runs three tenths fewer tiles over groups.
+// A step with entries and with groups: 1,000 atoms 54.5 and 54.3 us, 2,100 58.2 and 57.5,
+// 4,200 64.4 and 62.6, 8,400 75.6 and 70.3, 12,600 89.2 and 80.2.
 constexpr double ENTRY_TILES = 16384.0;
 static int has_entry_list(int mixed, double tiles) { return mixed && tiles < ENTRY_TILES; }
 // Launches of this many chunks of such lists or more run a wave per chunk, others a
@@ -377,11 +379,12 @@ constexpr double ENTRY_WAVE_CHUNKS = 4096.0;
 
 // Tiles per pair-kernel work item, from the system at its creation alone: how FP32 sums
 // are cut must depend neither on the batch around a system nor, under a barostat, on
-// the box in which its list happened to be allocated again.  A wave runs an item's tiles one after the other,
-// so a list of few items is as slow as one item: 1,000 atoms (6,000 tiles) 15.2 us
-// with 32 tiles, 9.6 with 16, 6.7 with 8.  An item costs its clusters' loads and
-// two force flushes: 227,000 atoms (2.2 M tiles) 285 us with 32, 300 with 16, 376
-// with 8; 24 systems of 1,000 to 25,000 atoms 408, 420 and 452 us a step.
+// the box in which its list happened to be allocated again.  A wave runs an item's
+// tiles one after the other, so a list of few items is as slow as one item: 1,000 atoms
+// (6,000 tiles, mixed form with pair groups) 15.2 us with 32 tiles, 9.6 with 16, 6.7 with
+// 8.  An item costs its clusters' loads and two force flushes: 227,000 atoms (2.2 M
+// tiles) 285 us with 32, 300 with 16, 376 with 8; 24 systems of 1,000 to 25,000 atoms
+// 408, 420 and 452 us a step.
 static int pair_item_tiles(double tiles) { return tiles < 16384.0 ? MIN_ITEM_TILES : tiles < 65536.0 ? 16 : 32; }
 
 int System::alloc_device() {
